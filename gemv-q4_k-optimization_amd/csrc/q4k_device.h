@@ -319,32 +319,46 @@ __device__ __forceinline__ uint32_t fastdiv(uint32_t n, const FastDiv &f) {
 // 1.5 * 2^23: the sum is exact in its integer part for |y| < 2^22, so its low
 // mantissa bits hold rint(y) (round-to-nearest-even, like the add itself)
 // and subtracting the constant back gives it as a float.  Contraction is off
-// so y is rounded on its own before the add.
+// so y is rounded on its own before the add.  Every workgroup quantises the
+// whole activation, so the instructions per value count: the low bytes of
+// four sums are gathered by byte permutes (a q8 in [-127, 127] is the sum's
+// low byte), the distances from rint(y) go through one maximum (the IEEE 2019
+// one, which keeps a NaN, so a NaN takes the exact path) and one compare, and
+// the sum of the q8 is a dot product with ones: about 50 instructions per
+// eight values against 62 with an or, an add and a compare per value (1024 x
+// 4096 N=1 3.40 -> 3.32 us, 4096 x 4096 N=4 6.63 -> 6.57, 14336 x 4096 N=8
+// 14.92 -> 14.78).
 template <int V, int H>
 __device__ __forceinline__ bool quantize_pack(const float (&v)[V], float d, float rd, bool exact,
                                               uint32_t (&word)[V / 4], int (&hsum)[H]) {
 #pragma clang fp contract(off)
     constexpr float kMagic = 12582912.0f;  // 1.5 * 2^23
-    bool fast = true;
+    float far = 0.0f;  // the largest distance of a y from rint(y); NaN if any is
 #pragma unroll
-    for (int w = 0; w < V / 4; ++w) word[w] = 0;
+    for (int w = 0; w < V / 4; ++w) {
+        uint32_t q[4];  // the low bytes hold the q8
 #pragma unroll
-    for (int h = 0; h < H; ++h) hsum[h] = 0;
-#pragma unroll
-    for (int k = 0; k < V; ++k) {
-        int q;
-        if (exact) {
-            q = (int)roundf(v[k] / d);
-        } else {
-            const float y = v[k] * rd;
-            const float m = y + kMagic;
-            q = __builtin_bit_cast(int, m) - 0x4B400000;
-            fast = fast && fabsf(y - (m - kMagic)) <= 0.5f - 0x1p-14f;
+        for (int k = 0; k < 4; ++k) {
+            if (exact) {
+                q[k] = (uint32_t)(int)roundf(v[4 * w + k] / d);
+            } else {
+                const float y = v[4 * w + k] * rd;
+                const float m = y + kMagic;
+                q[k] = __builtin_bit_cast(uint32_t, m);
+                far = __builtin_elementwise_maximum(far, fabsf(y - (m - kMagic)));
+            }
         }
-        hsum[k * H / V] += q;
-        word[k / 4] |= (uint32_t)(q & 0xff) << (8 * (k % 4));
+        word[w] = __builtin_amdgcn_perm(__builtin_amdgcn_perm(q[3], q[2], 0x0c0c0400u),
+                                        __builtin_amdgcn_perm(q[1], q[0], 0x0c0c0400u), 0x05040100u);
     }
-    return fast;
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+        hsum[h] = 0;
+#pragma unroll
+        for (int w = h * (V / 4) / H; w < (h + 1) * (V / 4) / H; ++w)
+            hsum[h] = __builtin_amdgcn_sdot4((int)word[w], 0x01010101, hsum[h], false);
+    }
+    return far <= 0.5f - 0x1p-14f;
 }
 
 // The q8 of one lane's V values packed four to a dword, and the sums over
