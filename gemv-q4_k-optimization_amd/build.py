@@ -39,7 +39,7 @@ def build(verbose: bool = False, save_temps: bool = False) -> str:
     # the device sources compile in parallel (each instantiates many kernels)
     dev_objs, procs = [], []
     for src in ("q4k_gemv.hip", "q6k_gemv.hip", "q4k_sums.hip", "q6k_sums.hip", "q4k_short.hip", "q6k_short.hip",
-                "q4k_probe.hip"):
+                "q4k_mfma.hip", "q6k_mfma.hip", "q4k_probe.hip"):
         obj = os.path.join(BUILD, src.replace(".hip", ".o"))
         cmd = [hipcc, f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC",
                # no packed-FP32 instructions in device code

@@ -52,8 +52,8 @@ __global__ __launch_bounds__(256) void quantize_q8_1_kernel(const float *__restr
 #pragma unroll
         for (int k = 0; k < 4; ++k) v[k] = i0 + k < ne00 ? src[k] : 0.0f;
     }
-    float amax = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
-    amax = block_max<8>(amax);
+    bool lane_nan;
+    const float amax = block_max<8>(lane_amax(v, lane_nan));
     float t[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) t[k] = v[k] + swizzle_xor<4>(v[k]);
@@ -63,9 +63,8 @@ __global__ __launch_bounds__(256) void quantize_q8_1_kernel(const float *__restr
     for (int k = 0; k < 4; ++k) t[k] += dppf<kDppXor1>(t[k]);
     const float sum = (t[0] + t[2]) + (t[1] + t[3]);
     const float d = div127(amax);
-    uint32_t word[1] = {0u};
-    int qsum[1];
-    if (amax != 0.0f) quantize_values<4, 1>(v, d, __builtin_amdgcn_rcpf(d), word, qsum);
+    uint32_t word[1];
+    quantize_values(v, amax, d, lane_nan, word);
     uint8_t *out = vy + (col * nblk_col + blk) * kQ81Bytes;
     *reinterpret_cast<uint32_t *>(out + 4 + 4 * e) = word[0];
     if (e == 0) {
@@ -82,7 +81,7 @@ struct SumsParams {
     int32_t *sqq;      // [M][K/32] for this column
     int32_t *sq;       // [K/32] for this column
     int M, K, nb, G, qcol;
-    FastDiv nblk32;
+    FastDiv upc;
 };
 
 // One wave per (row, group): the GEMV's lane map, swizzled activation layout,
@@ -91,7 +90,7 @@ __global__ __launch_bounds__(256) void subblock_sums_kernel(SumsParams p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     int8_t *q8s = reinterpret_cast<int8_t *>(lds);
     float2 *dks = reinterpret_cast<float2 *>(lds + p.qcol);
-    stage_from_q8_1<kLayoutQ4K, 256>(p.y, 0, p.K, 1, p.nblk32, p.qcol, q8s, dks);
+    stage_from_q8_1<kLayoutQ4K, 256>(p.y, 0, p.K, 1, p.upc, p.qcol, q8s, dks);
     __syncthreads();
     GemvParams gp{};
     gp.w = p.w;
@@ -291,8 +290,7 @@ static bool use_mfma_ga(int64_t M, int64_t N, int64_t K) {
 // first round -- KS at most the S summation segments of a row (S = min(8,
 // the largest power of two <= the super-blocks per row), a function of K
 // alone, which fixes the summation order).
-static Geometry pick_geometry_mfma(const DeviceInfo &di, int64_t K, int64_t M, int nc, int owgs, int owaves,
-                                   bool ga = false) {
+static Geometry pick_geometry_mfma(const DeviceInfo &di, int64_t K, int64_t M, int nc, int owgs, bool ga = false) {
     Geometry g;
     const int max_lds = di.max_lds > 0 ? di.max_lds : 65536;
     const int cus = di.cus > 0 ? di.cus : 1;
@@ -307,13 +305,8 @@ static Geometry pick_geometry_mfma(const DeviceInfo &di, int64_t K, int64_t M, i
     g.rows_base = (int)(tiles / g.grid);
     g.rows_extra = (int)(tiles % g.grid);
     const int64_t nt = g.rows_base + (g.rows_extra ? 1 : 0);
-    g.waves = 16;  // measured faster than 8 where the kernel is chosen
-    if (owaves >= 1 && owaves <= 16) g.waves = owaves > 8 ? 16 : 8;
-    if (ga) {  // GA: its A operands in flight take 146 registers at 2 items
-        g.waves = 8;
-        const int os = g_ovr_slots.load();
-        g.slots = os == 2 || os == 4 ? os : 2;
-    }
+    g.waves = 8;  // 16 measured slower from few tiles on (14336 x 4096 N=8 14.2 against 13.6 us)
+    if (ga) g.slots = g_ovr_slots.load() == 4 ? 4 : 2;
     const int64_t nb = K / kQK;
     g.segs = 1;
     while (g.segs < kMfmaMaxSegs && 2 * g.segs <= nb) g.segs *= 2;
@@ -933,12 +926,12 @@ static Geometry pick_geometry(const DeviceInfo &di, int64_t K, int64_t M, int64_
     if (q81 && !fused && mats == 1 && N <= kMfmaCols &&
         (okern == 6 || (okern == 0 && use_mfma_ga(M, N, K) &&
                          !(use_mfma(M, N, K) && mfma_lds_bytes((int)K, (int)N, 16) <= max_lds))))
-        return pick_geometry_mfma(di, K, M, (int)N, owgs, owaves, true);
+        return pick_geometry_mfma(di, K, M, (int)N, owgs, true);
     if (!fused && mats == 1 && (okern == 4 || (okern == 0 && use_mfma(M, N, K)))) {
         int mc = (int)N;
         while (mc > 1 && mfma_lds_bytes((int)K, mc, 16) > max_lds) mc = (mc + 1) / 2;
         if (mfma_lds_bytes((int)K, mc, 16) <= max_lds && (okern == 4 || mc == N))
-            return pick_geometry_mfma(di, K, M, mc, owgs, owaves);
+            return pick_geometry_mfma(di, K, M, mc, owgs);
     }
     g.grid = owgs > 0 ? owgs : grid_per_matrix(cus, mats, M);
     // One column with rows of at most 8192 values and ~500 KB or more of
@@ -1041,7 +1034,8 @@ static Geometry pick_geometry(const DeviceInfo &di, int64_t K, int64_t M, int64_
         g.lds_launch = max_lds / 2 + 256;
     // weight loads before quantisation only when every activation load fits
     // the staging rounds issued ahead of them
-    const bool pro0_ok = (int64_t)nc * (K / 32) <= (int64_t)stage_capacity(stage_lpb(nc), g.waves * kWave, nc);
+    const bool pro0_ok = (nc == 1 ? K / 32 : (int64_t)nc * stage_units((int)K) * 16) <=
+                         (int64_t)stage_capacity(stage_lpb(nc), g.waves * kWave, nc);
     g.prologue = pro0_ok ? 0 : 1;
     // One column and two slots on streams of under 8 steps per wave: one
     // early group instead of two (measured on MI355X: 4096 x 14336 9.06 ->
@@ -1150,46 +1144,6 @@ static const void *gemv_kernel_for(int nc, int R, int waves, int pro, int slots)
     return slots == 4 ? gemv_sym_r<16, 4>(nc, R, pro) : gemv_sym_r<16, 2>(nc, R, pro);
 }
 
-template <int WAVES>
-static const void *mfma_kernel_nc(int nc) {
-    switch (nc) {
-        case 1: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<1, WAVES>);
-        case 2: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<2, WAVES>);
-        case 3: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<3, WAVES>);
-        case 4: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<4, WAVES>);
-        case 5: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<5, WAVES>);
-        case 6: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<6, WAVES>);
-        case 7: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<7, WAVES>);
-        case 8: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<8, WAVES>);
-        default: return nullptr;
-    }
-}
-
-static const void *mfma_kernel_for(int nc, int waves) {
-    return waves > 8 ? mfma_kernel_nc<16>(nc) : mfma_kernel_nc<8>(nc);
-}
-
-template <int NIF>
-static const void *mfma_ga_kernel_nc(int nc) {
-    switch (nc) {
-        case 1: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<1, 8, false, true, NIF>);
-        case 2: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<2, 8, false, true, NIF>);
-        case 3: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<3, 8, false, true, NIF>);
-        case 4: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<4, 8, false, true, NIF>);
-        case 5: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<5, 8, false, true, NIF>);
-        case 6: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<6, 8, false, true, NIF>);
-        case 7: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<7, 8, false, true, NIF>);
-        case 8: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<8, 8, false, true, NIF>);
-        default: return nullptr;
-    }
-}
-
-// GA: 8-wave workgroups, 2 or 4 items in flight per wave
-static const void *mfma_ga_kernel_for(int nc, int waves, int nif) {
-    if (waves != 8) return nullptr;
-    return nif == 4 ? mfma_ga_kernel_nc<4>(nc) : mfma_ga_kernel_nc<2>(nc);
-}
-
 static int launch_gemv(DeviceInfo *di, const Geometry &geo, GemvParams p, int nc, hipStream_t stream,
                        const BatchLaunch *bl = nullptr) {
     const void *fn = nullptr;
@@ -1272,8 +1226,8 @@ static int launch_gemv(DeviceInfo *di, const Geometry &geo, GemvParams p, int nc
     } else if (geo.mfma) {
         if (geo.mfma_ga && (p.x || !p.y)) return Q4K_EINVAL;  // GA reads the Q8_1 buffer
         fn = geo.mfma_ga ? (p.sums ? q4k_mfma_ga_sums_kernel(nc, geo.waves, geo.slots)
-                                   : mfma_ga_kernel_for(nc, geo.waves, geo.slots))
-                         : (p.sums ? q4k_mfma_sums_kernel(nc, geo.waves) : mfma_kernel_for(nc, geo.waves));
+                                   : q4k_mfma_ga_kernel(nc, geo.waves, geo.slots))
+                         : q4k_mfma_kernel(nc, p.sums != nullptr);
         p.rows_base = geo.rows_base;
         p.rows_extra = geo.rows_extra;
         p.rpw = geo.ks;
@@ -1374,7 +1328,7 @@ static int run_gemv(const void *src0, int64_t ne00, int64_t ne01, int64_t nb01, 
         p.G = (p.nb + 15) / 16;
         p.qcol = q8_col_bytes((int)ne00);
         p.ntiles = geo.ntiles;
-        p.nblk32 = fastdiv_init((uint32_t)(ne00 / 32));
+        p.upc = fastdiv_init((uint32_t)stage_units((int)ne00));
         if (so) {  // parity variant: each column's launch on its own, same geometry and kernel
             for (int64_t c = 0; c < ncols; ++c) {
                 GemvParams pc = p;
@@ -1432,7 +1386,7 @@ static int run_gemv(const void *src0, int64_t ne00, int64_t ne01, int64_t nb01, 
         p.qcol = q8_col_bytes((int)ne00);
         p.ntiles = geo.ntiles;
         p.vec_ok = x && aligned(p.x, 16) && (ldx % 4 == 0);
-        p.nblk32 = fastdiv_init((uint32_t)(ne00 / 32));
+        p.upc = fastdiv_init((uint32_t)stage_units((int)ne00));
         if (fused) {
             p.gate = ep->gate;
             p.bias = ep->bias;
@@ -1842,7 +1796,7 @@ int q4k_subblock_sums(const void *src0, int64_t ne00, int64_t ne01, int64_t nb01
         p.nb = nb;
         p.G = (nb + 15) / 16;
         p.qcol = q8_col_bytes((int)ne00);
-        p.nblk32 = fastdiv_init((uint32_t)(ne00 / 32));
+        p.upc = fastdiv_init((uint32_t)stage_units((int)ne00));
         const int64_t items = ne01 * p.G;
         int grid = (int)((items + 3) / 4);
         if (grid > di->cus * 8) grid = di->cus * 8;

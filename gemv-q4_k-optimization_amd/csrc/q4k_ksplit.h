@@ -57,22 +57,14 @@ template <int V>
 __device__ __forceinline__ void ks_quantize_part(const float (&v)[V], uint32_t (&word)[V / 4], float &d8,
                                                  int &qsum, int &hsum) {
     constexpr int LPB = 32 / V;
-    float amax = 0.0f;
-#pragma unroll
-    for (int k = 0; k < V; ++k) amax = fmaxf(amax, fabsf(v[k]));
+    bool lane_nan;
+    float amax = lane_amax(v, lane_nan);
     if constexpr (LPB >= 2) amax = dpp_max_xor1(amax);
     if constexpr (LPB >= 4) amax = dpp_max_xor2(amax);
     if constexpr (LPB >= 8) amax = dpp_max_half_mirror(amax);
     const float d = div127(amax);
-    int s[1];
-    if (amax != 0.0f) {
-        quantize_values<V, 1>(v, d, __builtin_amdgcn_rcpf(d), word, s);
-    } else {
-#pragma unroll
-        for (int w = 0; w < V / 4; ++w) word[w] = 0;
-        s[0] = 0;
-    }
-    int t = s[0];
+    quantize_values(v, amax, d, lane_nan, word);
+    int t = packed_sum(word);
     if constexpr (LPB >= 4) t += dpp<kDppXor1>(t);
     if constexpr (LPB >= 8) t += dpp<kDppXor2>(t);
     hsum = t;

@@ -77,7 +77,6 @@ struct SumsOut {
 // automatic geometry picks for plain products are).
 const void *q4k_sums_kernel(int nc, int waves, int pro, int slots);
 const void *q4k_bpl_sums_kernel(int waves);
-const void *q4k_mfma_sums_kernel(int nc, int waves);
 const void *q4k_ksplit_sums_kernel(int sbw, int waves, int slots, int G);
 const void *q4k_ksplit_long_sums_kernel(int sbw, int waves, int slots, int G);
 const void *q4k_ksplit_nc_sums_kernel(int nc, int sbw, int waves, int slots, int G, bool staged);
@@ -89,6 +88,14 @@ const void *q6k_ksplit_long_sums_kernel(int sbw, int waves, int slots, int G);
 const void *q6k_ksplit_nc_sums_kernel(int nc, int p, int sbw, int waves, int slots);
 const void *q6k_mfma_ga_sums_kernel(int nc, int waves);
 const void *q6k_sums_kernel(int nc, int waves, int pro, int slots, bool dense);
+
+// The matrix-core kernels (q4k_mfma.hip, q6k_mfma.hip) for nc columns
+// (sums: the parity variant); ga: the A operand from the Q8_1 buffer, nif
+// items in flight per wave.
+const void *q4k_mfma_kernel(int nc, bool sums);
+const void *q4k_mfma_ga_kernel(int nc, int waves, int nif);
+const void *q6k_mfma_kernel(int nc, int waves);
+const void *q6k_mfma_ga_kernel(int nc, int waves);
 
 // The long-row K-split kernels with short teams (q4k_short.hip): the variant
 // of the launch shape and kind given (sums: the parity variant; epi:

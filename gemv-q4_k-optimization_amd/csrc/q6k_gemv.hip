@@ -26,14 +26,14 @@ struct Q6SumsParams {
     const uint8_t *y;  // one column of AoS Q8_1
     int32_t *s16;      // [M][K/16] for this column
     int M, K, nb, G, qcol;
-    FastDiv nblk32;
+    FastDiv upc;
 };
 
 __global__ __launch_bounds__(256) void q6_group_sums_kernel(Q6SumsParams p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     int8_t *q8s = reinterpret_cast<int8_t *>(lds);
     uint8_t *aux = lds + p.qcol;
-    stage_from_q8_1<kLayoutQ6K, 256>(p.y, 0, p.K, 1, p.nblk32, p.qcol, q8s, aux);
+    stage_from_q8_1<kLayoutQ6K, 256>(p.y, 0, p.K, 1, p.upc, p.qcol, q8s, aux);
     __syncthreads();
     GemvParams gp{};
     gp.K = p.K;
@@ -565,7 +565,8 @@ static Q6Geometry pick_geometry_q6(const DeviceInfo &di, int64_t K, int64_t M, i
     g.lds = q6_tile_lds_bytes((int)K, nc, g.waves, g.dense);
     g.lds_launch = g.lds;
     if (owgs == 0 && g.lds_launch <= max_lds / 2) g.lds_launch = max_lds / 2 + 256;
-    const bool pro0_ok = (int64_t)nc * (K / 32) <= (int64_t)stage_capacity(stage_lpb(nc), g.waves * kWave, nc);
+    const bool pro0_ok = (nc == 1 ? K / 32 : (int64_t)nc * stage_units((int)K) * 16) <=
+                         (int64_t)stage_capacity(stage_lpb(nc), g.waves * kWave, nc);
     g.prologue = pro0_ok ? 0 : 1;
     const int opro = g_ovr_prologue.load();
     if (opro == 1 || (opro == 0 && pro0_ok)) g.prologue = opro;
@@ -625,41 +626,6 @@ static const void *q6_kernel_for(int nc, int waves, int pro, int slots, int fuse
     }
     if (waves <= 8) return slots == 1 ? q6_sym_nc<8, 1, BATCH>(nc, pro) : q6_sym_nc<8, 2, BATCH>(nc, pro);
     return slots == 1 ? q6_sym_nc<16, 1, BATCH>(nc, pro) : q6_sym_nc<16, 2, BATCH>(nc, pro);
-}
-
-template <int WAVES>
-static const void *q6_mfma_kernel_nc(int nc) {
-    switch (nc) {
-        case 1: return reinterpret_cast<const void *>(&gemv_q6k_mfma_kernel<1, WAVES>);
-        case 2: return reinterpret_cast<const void *>(&gemv_q6k_mfma_kernel<2, WAVES>);
-        case 3: return reinterpret_cast<const void *>(&gemv_q6k_mfma_kernel<3, WAVES>);
-        case 4: return reinterpret_cast<const void *>(&gemv_q6k_mfma_kernel<4, WAVES>);
-        case 5: return reinterpret_cast<const void *>(&gemv_q6k_mfma_kernel<5, WAVES>);
-        case 6: return reinterpret_cast<const void *>(&gemv_q6k_mfma_kernel<6, WAVES>);
-        case 7: return reinterpret_cast<const void *>(&gemv_q6k_mfma_kernel<7, WAVES>);
-        case 8: return reinterpret_cast<const void *>(&gemv_q6k_mfma_kernel<8, WAVES>);
-        default: return nullptr;
-    }
-}
-
-static const void *q6_mfma_kernel_for(int nc, int waves) {
-    return waves > 8 ? q6_mfma_kernel_nc<16>(nc) : q6_mfma_kernel_nc<8>(nc);
-}
-
-// GA: 8-wave workgroups
-static const void *q6_mfma_ga_kernel_for(int nc, int waves) {
-    if (waves != 8) return nullptr;
-    switch (nc) {
-        case 1: return reinterpret_cast<const void *>(&gemv_q6k_mfma_kernel<1, 8, false, true>);
-        case 2: return reinterpret_cast<const void *>(&gemv_q6k_mfma_kernel<2, 8, false, true>);
-        case 3: return reinterpret_cast<const void *>(&gemv_q6k_mfma_kernel<3, 8, false, true>);
-        case 4: return reinterpret_cast<const void *>(&gemv_q6k_mfma_kernel<4, 8, false, true>);
-        case 5: return reinterpret_cast<const void *>(&gemv_q6k_mfma_kernel<5, 8, false, true>);
-        case 6: return reinterpret_cast<const void *>(&gemv_q6k_mfma_kernel<6, 8, false, true>);
-        case 7: return reinterpret_cast<const void *>(&gemv_q6k_mfma_kernel<7, 8, false, true>);
-        case 8: return reinterpret_cast<const void *>(&gemv_q6k_mfma_kernel<8, 8, false, true>);
-        default: return nullptr;
-    }
 }
 
 int check_weight_q6(const void *src0, int64_t ne00, int64_t ne01, int64_t nb01) {
@@ -758,7 +724,7 @@ int run_gemv_q6(const void *src0, int64_t ne00, int64_t ne01, int64_t nb01, cons
         p.rows_base = geo.rows_base;
         p.rows_extra = geo.rows_extra;
         p.ring_off = q6_act_bytes(p.K, nc, dense);
-        p.nblk32 = fastdiv_init((uint32_t)(ne00 / 32));
+        p.upc = fastdiv_init((uint32_t)stage_units((int)ne00));
         if (fused) {
             p.gate = ep->gate;
             p.bias = ep->bias;
@@ -782,8 +748,8 @@ int run_gemv_q6(const void *src0, int64_t ne00, int64_t ne01, int64_t nb01, cons
                              ? q6_ksplit_kernel_epi<kEpiBias>(geo.ks_long != 0, geo.ksplit, geo.waves, geo.slots, p.G)
                          : geo.ks_long  ? q6_ksplit_long_kernel<false>(geo.ksplit, geo.waves, geo.slots, p.G)
                          : geo.ksplit ? q6_ksplit_kernel<false>(geo.ksplit, geo.waves, geo.slots, p.G)
-                         : geo.mfma_ga ? q6_mfma_ga_kernel_for(nc, geo.waves)
-                         : geo.mfma ? q6_mfma_kernel_for(nc, geo.waves)
+                         : geo.mfma_ga ? q6k_mfma_ga_kernel(nc, geo.waves)
+                         : geo.mfma ? q6k_mfma_kernel(nc, geo.waves)
                          : bl       ? q6_kernel_for<true>(nc, geo.waves, geo.prologue, geo.slots, fused, dense)
                                     : q6_kernel_for<false>(nc, geo.waves, geo.prologue, geo.slots, fused, dense);
         const bool several = geo.ks_nc_p || geo.ks_snc;
@@ -963,7 +929,7 @@ int q6k_group_sums(const void *src0, int64_t ne00, int64_t ne01, int64_t nb01, c
         p.nb = nb;
         p.G = (nb + 15) / 16;
         p.qcol = q8_col_bytes((int)ne00);
-        p.nblk32 = fastdiv_init((uint32_t)(ne00 / 32));
+        p.upc = fastdiv_init((uint32_t)stage_units((int)ne00));
         const int64_t items = ne01 * p.G;
         int grid = (int)((items + 3) / 4);
         if (grid > di->cus * 8) grid = di->cus * 8;

@@ -346,18 +346,29 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q6k_mfma_kernel(Q4K_GEMV_KE
     int8_t *q8s = reinterpret_cast<int8_t *>(lds);
     float *dks = reinterpret_cast<float *>(lds + q6m_dk_off(p.K, NC));
 
+    constexpr int kLPB = stage_lpb(NC);
+    constexpr int kPreR = GA ? 1 : pre_rounds(NC, NT);
+    ActStage<kLPB, kPreR> xs;
+    Q81Stage<kPreR> ys;
+    if constexpr (!GA) {
+        // first of all: everything waits for the activation
+        if (p.x) stage_f32_issue<kLPB, NT>(p.x, p.ldx, p.K, NC, p.vec_ok != 0, p.upc, xs);
+        else stage_q81_issue<NT>(p.y, p.stride_col_y, p.K, NC, p.upc, ys);
+        __builtin_amdgcn_sched_barrier(0);
+    }
     Q6MLane ln = q6m_lane<NC, GA>(p.K, p.stride_col_y);
     q6m_chunks(ln, p.row_stride);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int KS = p.rpw, S = p.ntiles;
-    const int group = wave / KS, ks = wave - group * KS;
-    const int ngroups = WAVES / KS;
-    const int segs = S / KS, seg0 = ks * segs;  // the wave's run of segments
+    // KS and S are powers of two
+    const int KS = p.rpw, lks = __builtin_ctz(KS), S = p.ntiles, ls = __builtin_ctz(S);
+    const int group = wave >> lks, ks = wave & (KS - 1);
+    const int ngroups = WAVES >> lks;
+    const int segs = S >> lks, seg0 = ks * segs;  // the wave's run of segments
     const int b = (int)blockIdx.x;
     const int t0 = b * p.rows_base + min(b, p.rows_extra);
     const int nt = p.rows_base + (b < p.rows_extra ? 1 : 0);
-    const int rounds = (nt + ngroups - 1) / ngroups;
-    const int kb0 = seg0 * p.nb / S, kb1 = (seg0 + segs) * p.nb / S;  // kb1 > kb0 (S <= nb)
+    const int rounds = (nt + ngroups - 1) * KS / WAVES;
+    const int kb0 = seg0 * p.nb >> ls, kb1 = (seg0 + segs) * p.nb >> ls;  // kb1 > kb0 (S <= nb)
     const int items = rounds * (kb1 - kb0);
     const int row0 = t0 * kMfmaRows;
     const int nrows = min(nt * kMfmaRows, p.M - row0);
@@ -365,15 +376,7 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q6k_mfma_kernel(Q4K_GEMV_KE
         make_rsrc(p.w + (int64_t)row0 * p.row_stride, nrows > 0 ? (uint32_t)(nrows * p.row_stride) : 0u);
 
     constexpr int NQ = NC > 4 ? 2 : 1;
-    constexpr int kLPB = stage_lpb(NC);
-    constexpr int kPreR = GA ? 1 : pre_rounds(NC, NT);
-    ActStage<kLPB, kPreR> xs;
-    Q81Stage<kPreR> ys;
-    if constexpr (!GA) {
-        if (p.x) stage_f32_issue<kLPB, NT>(p.x, p.ldx, p.K, NC, p.vec_ok != 0, p.nblk32, xs);
-        else stage_q81_issue<NT>(p.y, p.stride_col_y, p.K, NC, p.nblk32, ys);
-        __syncthreads();  // all activation loads of this CU are queued first
-    }
+    if constexpr (!GA) __syncthreads();  // all activation loads of this CU are queued first
     const __amdgpu_buffer_rsrc_t ry =
         make_rsrc(p.y, GA ? (uint32_t)((int64_t)(NC - 1) * p.stride_col_y * kQ81Bytes + (p.K / 32) * kQ81Bytes) : 0u);
 
@@ -410,10 +413,10 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q6k_mfma_kernel(Q4K_GEMV_KE
             reinterpret_cast<u32x4 *>(lds + q6m_ga_zero_off(p.K))[threadIdx.x] = u32x4{0u, 0u, 0u, 0u};
     } else {
         if (p.x)
-            stage_f32_finish<kLayoutMfmaQ6, kLPB, NT>(p.x, p.ldx, p.K, NC, p.vec_ok != 0, p.nblk32, xs,
+            stage_f32_finish<kLayoutMfmaQ6, kLPB, NT>(p.x, p.ldx, p.K, NC, p.vec_ok != 0, p.upc, xs,
                                                       mfma_qcol(p.K), q8s, dks);
         else
-            stage_q81_finish<kLayoutMfmaQ6, NT>(p.y, p.stride_col_y, p.K, NC, p.nblk32, ys, mfma_qcol(p.K), q8s,
+            stage_q81_finish<kLayoutMfmaQ6, NT>(p.y, p.stride_col_y, p.K, NC, p.upc, ys, mfma_qcol(p.K), q8s,
                                                 dks);
         // the zero area of the A operand, and d8 of the padding columns (their
         // outputs are dropped; zeros keep them finite)
@@ -438,7 +441,7 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q6k_mfma_kernel(Q4K_GEMV_KE
     const uint8_t *const pa[2] = {GA && ln.a_data[0] ? aslot + ln.ar_off[0] : lds + q6m_ga_zero_off(p.K),
                                   GA && ln.a_data[1] ? aslot + ln.ar_off[1] : lds + q6m_ga_zero_off(p.K)};
     int t = 0;                            // local segment of the current item
-    int seg_end = (seg0 + 1) * p.nb / S;  // its end (super-block)
+    int seg_end = (seg0 + 1) * p.nb >> ls;  // its end (super-block)
     // items go two at a time (load slot k holds item it); an odd count ends
     // with one item past the wave's, whose zeros add nothing
     for (int it = 0; it < items;) {
@@ -467,12 +470,12 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q6k_mfma_kernel(Q4K_GEMV_KE
                 q6m_tree_push(t, v, l1, l2, l4);
                 ++t;
                 if (t < segs) {
-                    seg_end = (seg0 + t + 1) * p.nb / S;
+                    seg_end = (seg0 + t + 1) * p.nb >> ls;
                     continue;
                 }
                 // round end: v is the wave's subtree of the tile
                 t = 0;
-                seg_end = (seg0 + 1) * p.nb / S;
+                seg_end = (seg0 + 1) * p.nb >> ls;
                 const int buf = done.r & 1;
                 *reinterpret_cast<float2 *>(part + ((buf * WAVES + wave) * 64 + ln.lane) * 2) = make_float2(v[0], v[1]);
                 __syncthreads();
