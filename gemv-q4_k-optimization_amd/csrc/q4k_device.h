@@ -197,7 +197,7 @@ __device__ __forceinline__ int byte_sum16(u32x4 a) {
 //             (d8 is a half widened), so a lane reads those of four
 //             consecutive columns in one 8-byte read, then d8 * sum q8 as
 //             floats, km[8b + c] from K / 2 bytes on.
-//   MFMA Q6   the MFMA layout with d8 alone as the auxiliary term, d8[8b + c]
+//   MFMA Q6   the MFMA layout with d8 alone (half) as the auxiliary term, d8[8b + c]
 //             (the Q6_K matrix-core kernel folds the -32 offset into its
 //             weight bytes, so it needs no activation sums).
 //
@@ -216,7 +216,7 @@ constexpr int kLayoutQ4K = 1;
 constexpr int kLayoutQ6K = 2;
 constexpr int kLayoutQ6KDense = 3;
 constexpr int kLayoutMfma = 4;  // linear q8 columns; d8 (half), then d8*sum per [block][column] of 8 columns
-constexpr int kLayoutMfmaQ6 = 5;  // linear q8 columns; d8 per [block][column] of 8 columns
+constexpr int kLayoutMfmaQ6 = 5;  // linear q8 columns; d8 (half) per [block][column] of 8 columns
 constexpr int kLayoutQ4KS2 = 6;   // Q4K, positions permuted for the two-column K-split tree
 constexpr int kLayoutQ4KS4 = 7;   // Q4K, positions permuted for the four-column K-split tree
 constexpr int kLayoutQ6KS2 = 8;   // Q6K, positions permuted for the two-column K-split tree
@@ -300,7 +300,7 @@ __device__ __forceinline__ void store_aux(void *aux, int a0, int a1, int half, f
             reinterpret_cast<float *>(aux)[a1] = d8 * (float)qsum;
         }
     } else if (LAYOUT == kLayoutMfmaQ6) {
-        if (half == 0) reinterpret_cast<float *>(aux)[a0] = d8;
+        if (half == 0) reinterpret_cast<_Float16 *>(aux)[a0] = (_Float16)d8;
     } else if (half == 0) {
         reinterpret_cast<float2 *>(aux)[a0] = make_float2(d8, d8 * (float)qsum);
     }
@@ -324,76 +324,6 @@ __host__ __device__ inline FastDiv fastdiv_init(uint32_t d) {
 
 __device__ __forceinline__ uint32_t fastdiv(uint32_t n, const FastDiv &f) {
     return (__umulhi(n, f.mul) + n) >> f.shift;
-}
-
-// The q8 of one lane's V values of a block, packed four to a dword: q[k] =
-// roundf(v[k] / d) with the correctly rounded quotient, as ggml-cuda's
-// quantize_q8_1 computes it (0 where the block's amax is 0); amax is the
-// block's, d = amax / 127, lane_nan: the lane has a NaN among its values.
-//
-// Every workgroup quantises the whole activation before its first product, so
-// the instructions per value count.  r = rcp(d) is within 2^-22 of 1/d
-// (v_rcp_f32 is 1-ulp accurate), so v / d lies between v r (1 - 2^-20) and
-// v r (1 + 2^-20), and so does its rounded value.  One fma for each of the
-// two bounds adds 1.5 * 2^23, which rounds to the integer (ties to even) and
-// leaves it in the low mantissa bits: where the two agree no half-integer lies
-// between the bounds (or on one: they would differ, or v is 0) and the low
-// byte is the answer.  A lane with a value where they differ (one in ~10^4),
-// with a NaN, or of a block whose amax is so small that r could overflow,
-// recomputes its values with the exact division (an infinite amax: d is a NaN
-// and every byte 0, as from the division).  So a value takes two fmas, one bit
-// operation that collects the differences and 3/4 of a byte permute (a q8 in
-// [-127, 127] is the sum's low byte).
-template <int V>
-__device__ __forceinline__ void quantize_values(const float (&v)[V], float amax, float d, bool lane_nan,
-                                                uint32_t (&word)[V / 4]) {
-#pragma clang fp contract(off)
-    constexpr float kMagic = 12582912.0f;  // 1.5 * 2^23
-    const float r = __builtin_amdgcn_rcpf(d);
-    const float r0 = r * (1.0f - 0x1p-20f), r1 = r * (1.0f + 0x1p-20f);
-    uint32_t differ = 0;
-#pragma unroll
-    for (int w = 0; w < V / 4; ++w) {
-        uint32_t q[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const float x = v[4 * w + k];
-            q[k] = __builtin_bit_cast(uint32_t, __builtin_fmaf(x, r0, kMagic));
-            // differ |= q ^ the other (as one instruction; the compiler would
-            // turn the collected bits back into a compare per value)
-            differ = __builtin_amdgcn_bitop3_b32(
-                differ, q[k], __builtin_bit_cast(uint32_t, __builtin_fmaf(x, r1, kMagic)), 0xF6);
-        }
-        word[w] = __builtin_amdgcn_perm(__builtin_amdgcn_perm(q[3], q[2], 0x0c0c0400u),
-                                        __builtin_amdgcn_perm(q[1], q[0], 0x0c0c0400u), 0x05040100u);
-    }
-    if (__builtin_expect(differ != 0 || lane_nan || !(amax >= 0x1p-100f), 0)) {
-#pragma unroll
-        for (int w = 0; w < V / 4; ++w) {
-            word[w] = 0;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int q = amax == 0.0f ? 0 : (int)roundf(v[4 * w + k] / d);
-                word[w] |= (uint32_t)(q & 0xff) << (8 * k);
-            }
-        }
-    }
-}
-
-// The largest |v| of a lane's values, NaNs left out (as by fmaxf), and whether
-// there are any.
-template <int V>
-__device__ __forceinline__ float lane_amax(const float (&v)[V], bool &has_nan) {
-    float a = 0.0f;
-#pragma unroll
-    for (int k = 0; k < V; ++k) a = __builtin_elementwise_maximum(a, fabsf(v[k]));  // keeps a NaN
-    has_nan = a != a;
-    if (__builtin_expect(has_nan, 0)) {
-        a = 0.0f;
-#pragma unroll
-        for (int k = 0; k < V; ++k) a = fmaxf(a, fabsf(v[k]));
-    }
-    return a;
 }
 
 // The sum of the q8 in a lane's packed dwords.
@@ -487,10 +417,95 @@ Q4K_DPP_MAX(half_mirror)
 // Reductions over the LPB lanes of a 32-value block (aligned lane groups).
 template <int LPB>
 __device__ __forceinline__ float block_max(float v) {
-    v = dpp_max_xor1(v);
-    v = dpp_max_xor2(v);
-    if (LPB == 8) v = dpp_max_half_mirror(v);
+    if (LPB >= 2) v = dpp_max_xor1(v);
+    if (LPB >= 4) v = dpp_max_xor2(v);
+    if (LPB >= 8) v = dpp_max_half_mirror(v);
     return v;
+}
+
+// The largest |v| of a lane's values: without the NaNs, as by fmaxf, or (KEEP)
+// NaN where there are any; chains of up to 8 values, which overlap.
+template <bool KEEP, int V>
+__device__ __forceinline__ float lane_amax(const float (&v)[V]) {
+    constexpr int kChains = V > 8 ? 2 : 1;
+    float a[kChains];
+#pragma unroll
+    for (int h = 0; h < kChains; ++h) {
+        a[h] = 0.0f;
+#pragma unroll
+        for (int k = h * (V / kChains); k < (h + 1) * (V / kChains); ++k)
+            a[h] = KEEP ? __builtin_elementwise_maximum(a[h], fabsf(v[k])) : fmaxf(a[h], fabsf(v[k]));
+    }
+    if (kChains == 1) return a[0];
+    return KEEP ? __builtin_elementwise_maximum(a[0], a[kChains - 1]) : fmaxf(a[0], a[kChains - 1]);
+}
+
+// The quantisation of a 32-value block by its 32 / V lanes, as ggml-cuda's
+// quantize_q8_1: d = amax / 127 and the lane's V q8, packed four to a dword:
+// roundf(v[k] / d) with the correctly rounded quotient (0 where amax is 0).
+//
+// Every workgroup quantises the whole activation before its first product, so
+// the instructions per value count, and where few waves share a SIMD the
+// length of the dependent chain too.  r = rcp(d) is 1-ulp accurate, so within
+// 2^-23 of 1/d; the two bounds r0 and r1, 1.25 and 1.5 * 2^-22 below and above
+// it, allow for that, for their own rounding (2^-24) and for the quotient's
+// (2^-24): v / d lies between v r0 and v r1, and so does its rounded value.
+// One fma for each bound adds 1.5 * 2^23, which rounds to the integer (ties to
+// even) and leaves it in the low mantissa bits: where the two agree no
+// half-integer lies between the bounds (or on one: they would differ, or v is
+// 0) and the low byte is the answer (a q8 in [-127, 127] is the sum's low
+// byte).  So a value takes two fmas, one bit operation that collects the
+// differences (a chain per dword) and 3/4 of a byte permute.  A block of zeros
+// passes: 0 * inf is the default NaN, low byte 0.  Where a lane of the wave has
+// a value whose bounds differ (one value in ~4 * 10^4), a NaN, or an amax so
+// small that r could overflow, the wave starts again with the exact division
+// (an infinite amax: d is a NaN and every byte 0 either way).  Bounds 8 * 2^-22
+// apart, which a workgroup of 4096 values left every third time, cost 0.2 to
+// 0.4 us (1024 x 16384 6.83 against 6.47 us, 4096 x 4096 N=4 6.50 / 6.30).
+template <int V>
+__device__ __forceinline__ void quantize_lanes(const float (&v)[V], float &d, uint32_t (&word)[V / 4]) {
+#pragma clang fp contract(off)
+    constexpr int LPB = 32 / V;
+    constexpr float kMagic = 12582912.0f;  // 1.5 * 2^23
+    const float lane_max = lane_amax<true>(v);
+    const float amax = block_max<LPB>(lane_max);  // (without the lanes that hold a NaN)
+    d = div127(amax);
+    const float r = __builtin_amdgcn_rcpf(d);
+    const float r0 = r * (1.0f - 0x1.4p-22f), r1 = r * (1.0f + 0x1.8p-22f);
+    uint32_t differ[V / 4];
+#pragma unroll
+    for (int w = 0; w < V / 4; ++w) {
+        uint32_t q[4];
+        differ[w] = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float x = v[4 * w + k];
+            q[k] = __builtin_bit_cast(uint32_t, __builtin_fmaf(x, r0, kMagic));
+            // differ |= q ^ the other (as one instruction; the compiler would
+            // turn the collected bits back into a compare per value)
+            differ[w] = __builtin_amdgcn_bitop3_b32(
+                differ[w], q[k], __builtin_bit_cast(uint32_t, __builtin_fmaf(x, r1, kMagic)), 0xF6);
+        }
+        word[w] = __builtin_amdgcn_perm(__builtin_amdgcn_perm(q[3], q[2], 0x0c0c0400u),
+                                        __builtin_amdgcn_perm(q[1], q[0], 0x0c0c0400u), 0x05040100u);
+    }
+    uint32_t any = differ[0];
+#pragma unroll
+    for (int w = 1; w < V / 4; ++w) any |= differ[w];
+    // 0 < amax < 2^-100
+    const bool tiny = __builtin_bit_cast(uint32_t, amax) - 1u < __builtin_bit_cast(uint32_t, 0x1p-100f) - 1u;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(any != 0 || lane_max != lane_max || tiny) != 0, 0)) {
+        const float exact_max = block_max<LPB>(lane_amax<false>(v));
+        d = div127(exact_max);
+        const float dd = exact_max == 0.0f ? 1.0f : d;  // (then the values are zeros and NaNs)
+#pragma unroll
+        for (int w = 0; w < V / 4; ++w) {
+            word[w] = 0;
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                word[w] |= (uint32_t)((int)roundf(v[4 * w + k] / dd) & 0xff) << (8 * k);
+        }
+    }
 }
 
 // Integer sums over the LPB lanes of a 32-value block: `half` over the lanes
@@ -605,11 +620,9 @@ template <int LAYOUT, int LPB>
 __device__ __forceinline__ void quantize_block_part(const float (&v)[32 / LPB], int e, bool live, const StageDst &at,
                                                     int8_t *q8s, void *aux, int32_t *sq_out = nullptr) {
     constexpr int V = 32 / LPB;
-    bool lane_nan;
-    const float amax = block_max<LPB>(lane_amax(v, lane_nan));
-    const float d = div127(amax);
+    float d;
     uint32_t word[V / 4];
-    quantize_values(v, amax, d, lane_nan, word);
+    quantize_lanes(v, d, word);
     int hsum, fsum;
     block_sums<LPB>(packed_sum(word), hsum, fsum);
     if (!live) return;

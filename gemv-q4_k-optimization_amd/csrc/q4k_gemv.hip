@@ -29,7 +29,7 @@ namespace q4k {
 
 // F32 -> AoS block_q8_1 with ggml-cuda's quantize_q8_1 arithmetic (call site
 // kernels/mmvq.cu:728-735): per 32 values d = amax/127 (div127, the IEEE
-// quotient), q = roundf(x/d) (quantize_values), ds = (half(d), half(sum x)).
+// quotient), q = roundf(x/d) (quantize_lanes), ds = (half(d), half(sum x)).
 // Eight lanes per block, four values (one 16-byte load) per lane, 32 blocks
 // per 256-thread workgroup.  amax is order-free; the sum follows the tree of
 // ggml's 32-lane warp_reduce_sum (partners at element distance 16, 8, 4, 2,
@@ -52,8 +52,6 @@ __global__ __launch_bounds__(256) void quantize_q8_1_kernel(const float *__restr
 #pragma unroll
         for (int k = 0; k < 4; ++k) v[k] = i0 + k < ne00 ? src[k] : 0.0f;
     }
-    bool lane_nan;
-    const float amax = block_max<8>(lane_amax(v, lane_nan));
     float t[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) t[k] = v[k] + swizzle_xor<4>(v[k]);
@@ -62,9 +60,9 @@ __global__ __launch_bounds__(256) void quantize_q8_1_kernel(const float *__restr
 #pragma unroll
     for (int k = 0; k < 4; ++k) t[k] += dppf<kDppXor1>(t[k]);
     const float sum = (t[0] + t[2]) + (t[1] + t[3]);
-    const float d = div127(amax);
+    float d;
     uint32_t word[1];
-    quantize_values(v, amax, d, lane_nan, word);
+    quantize_lanes(v, d, word);
     uint8_t *out = vy + (col * nblk_col + blk) * kQ81Bytes;
     *reinterpret_cast<uint32_t *>(out + 4 + 4 * e) = word[0];
     if (e == 0) {
@@ -237,51 +235,63 @@ static int tile_lds_bytes(int K, int nc, int waves) {
 }
 static int lds_bytes_linear(int K) { return K + K / 4; }
 
-// Products that run on the matrix-core kernel when no override says
-// otherwise (all columns in one launch, which the caller checks).  Measured
-// on MI355X against the tile kernel (interleaved, one process; us):
-//  - rows of 4096 values: eight columns from 896 row tiles (14336 rows), six
-//    to eight from 4096 tiles: 128256 x 4096 N=8 64.5 against 83.4, N=6
-//    63.6 against 73.2; 28672 x 4096 N=8 21.1 against 22.9; 14336 x 4096 N=8
-//    14.1 against 15.7.  Slower with fewer rows (4096 x 4096 N=8 10.2
-//    against 8.6; 11008 x 4096 N=8 13.7 against 12.9) or fewer columns
-//    (14336 x 4096 N=6 13.8 against 13.3; 128256 x 4096 N=4 62.7 against
-//    57.6: padded columns cost scaling work).
-//  - longer rows (two or more 16-block groups, where the tile kernel reads
-//    every column's activation from LDS at each step): six to eight columns
-//    from 512 tiles, five from 864: 8192 x 8192 N=8 17.8 against 22.0, N=6
-//    17.0 against 19.4; 13824 x 5120 N=8 18.2 against 26.0, N=5 16.6 against
-//    18.0; 28672 x 10240 N=5 43.4 against 50.1.  Slower at 5120 x 5120 and
-//    below (N=7 13.0 against 12.5), at five columns of 8192 x 5120 or 6144
-//    (13.1 against 12.9) and at four columns (8192 x 8192 14.5 against 13.3).
-//  - shorter rows: the tile kernel (18944 x 3584 N=8 17.7 against 18.7).
-// Rows longer than ~10,700 values need two launches for eight columns and
-// are left to the tile kernel (4096 x 14336 N=8).  Four items in flight per
-// wave instead of two measured slower on every shape.
+// Where the automatic choice is the matrix-core kernel (us per op, MI355X,
+// matrix-core against the choice without it).  It costs the same from one to
+// eight columns, so it pays where the tile kernel's work per column, or the
+// lanes it leaves idle on rows shorter than 16 super-blocks, have grown past
+// that.
+//  - rows of one or two super-blocks (up to 512 values), which have no short
+//    teams: two columns and more from 256 row tiles: 65536 x 512 N=3 9.34
+//    against 22.1, 8192 x 512 N=2 4.55 / 5.45, 65536 x 256 N=2 7.15 / 17.5
+//    (2048 x 512 N=4 4.37 / 4.04: not with fewer).
+//  - rows of 3 to 13: five columns and more from 256 tiles: 65536 x 1024 N=8
+//    13.4 / 39.2, 32768 x 768 N=5 8.18 / 17.4, 4096 x 2048 N=6 5.43 / 6.44,
+//    24576 x 3328 N=5 16.9 / 17.2 (2048 x 768 N=6 5.42 / 4.41, 2048 x 2560 N=6
+//    6.14 / 5.77).  Three and four columns only from 9 super-blocks on (rows
+//    of 3 to 8 run in short teams there): four from 1024 tiles, three from
+//    2048: 16384 x 2304 N=4 9.39 / 10.5, 32768 x 2304 N=3 13.3 / 15.4 (8192 x
+//    3328 N=4 8.29 / 8.10, 16384 x 2560 N=3 9.39 / 9.27).
+//  - rows of 14 to 16: eight columns from 896 tiles and six to eight from 4096
+//    (14336 x 4096 N=8 13.1 / 16.6, 128256 x 4096 N=8 64.6 / 87.3); with fewer
+//    rows or columns the tile kernel is within a few percent either way
+//    (4096 x 4096 N=8 8.4 / 8.8, N=5 7.3 / 7.2; 14336 x 4096 N=4 11.8 / 10.9).
+//  - rows of up to 5120 values: six columns from 512 tiles, five from 864
+//    (13824 x 5120 N=6 15.0 / 20.9); of up to 8192 (where the tile kernel
+//    reads every column's activation from LDS at each step): six from just
+//    over 8 rows per CU, five from 512 tiles: 4096 x 8192 N=8 13.8 / 15.8, N=6
+//    13.0 / 13.7, 8192 x 6144 N=5 12.0 / 14.0 (3072 x 8192 N=5 11.4 / 11.2);
+//    longer ones as those of 5120: with fewer rows the kernel below is the
+//    better one (4096 x 11008 N=6 15.6 against 15.0).
+// Rows whose columns do not fit the LDS in one launch are left to the others.
 static bool use_mfma(int64_t M, int64_t N, int64_t K) {
     const int64_t tiles = (M + kMfmaRows - 1) / kMfmaRows;
-    if (K < 4096) return false;
-    if (K == 4096) return (N == 8 && tiles >= 896) || (N >= 6 && tiles >= 4096);
+    if (K <= 512) return N >= 2 && tiles >= 256;
+    if (K < 3584) {
+        if (N >= 5) return tiles >= 256;
+        return K >= 2304 && ((N == 4 && tiles >= 1024) || (N == 3 && tiles >= 2048));
+    }
+    if (K <= 4096) return K == 4096 && ((N == 8 && tiles >= 896) || (N >= 6 && tiles >= 4096));
+    if (K <= 5120) return (N >= 6 && tiles >= 512) || (N == 5 && tiles >= 864);
+    if (K <= 8192) return (N >= 6 && tiles > 128) || (N == 5 && tiles >= 512);
     return (N >= 6 && tiles >= 512) || (N == 5 && tiles >= 864);
 }
 
 // Where the pre-quantised route runs the matrix-core kernel with its A
-// operand read from the Q8_1 buffer (GA): rows longer than 8192 values,
-// five to eight columns, a tile per CU or more, where (the caller checks)
-// the staged matrix-core kernel is not chosen or cannot hold the columns.
-// Measured on MI355X (us per op with a Q8_1 workspace, the quantiser launch
-// included; GA against the tile kernel): 4096 x 14336 N=8 18.35 against
-// 22.84, N=6 17.66 / 19.86, N=5 17.38 / 18.16; 8192 x 28672 N=8 44.07 /
-// 66.95, N=6 42.65 / 62.90.  Slower at four columns (8192 x 28672 39.40 /
-// 37.62) and than the staged matrix-core kernel where that is chosen and
-// holds the columns (13824 x 5120 N=8 24.74 against 17.87, 8192 x 8192
-// N=8 17.54 / 17.34, 28672 x 4096 N=8 22.99 / 21.70).  Two items in flight
-// per wave, not four (4096 x 14336 N=8 18.35 against 20.07); weights
-// through the slot, not loaded straight into the lanes' registers in MFMA
-// order (4096 x 14336 N=6 17.57 against 21.43).
+// operand read from the Q8_1 buffer (GA): rows longer than 8192 values, five to
+// eight columns, more than 8 rows per CU (below, the column split), where (the
+// caller checks) the staged matrix-core kernel is not chosen or cannot hold
+// the columns.  Measured on MI355X (us per op with a Q8_1 workspace, the
+// quantiser launch included; GA against the tile kernel): 4096 x 14336 N=8
+// 18.7 against 23, 8192 x 28672 N=8 44 / 67; against the column split, 3072 x
+// 14336 N=7 17.2 / 23.5, 2432 x 9472 N=7 13.7 / 15.8, 3072 x 22272 N=7 22.9 /
+// 35.3, 3072 x 28672 N=5 25.2 / 30.8 (2048 x 14336 N=6 16.3 / 16.1, 1024 x
+// 22272 N=7 21.5 / 16.6: not with fewer rows).  Slower at four columns (8192 x
+// 28672 39.4 / 37.6).  Two items in flight per wave, not four (4096 x 14336
+// N=8 15.1 against 17.0, quantised before); weights through the slot, not
+// loaded straight into the lanes' registers in MFMA order (N=6 17.6 / 21.4).
 static bool use_mfma_ga(int64_t M, int64_t N, int64_t K) {
     const int64_t tiles = (M + kMfmaRows - 1) / kMfmaRows;
-    return K > 8192 && N >= 5 && tiles >= 256;
+    return K > 8192 && N >= 5 && tiles > 128;
 }
 
 // The matrix-core kernel: one workgroup per CU (at most one per tile) of 8
@@ -786,6 +796,9 @@ bool split_columns(int64_t K, int64_t M, int64_t N, int cus) {
     // 2048 N=3 4.81 / 4.26; at up to 4 the split: 512 x 2048 N=4 3.08 / 4.04,
     // 1024 x 2560 N=4 4.18 / 4.53)
     const int64_t lim = K < 4096 && K > 1024 ? 4 : (N == 2 ? 8 : 12);
+    // five columns or more of long rows: up to 8 rows per CU (beyond, the
+    // matrix-core kernels: use_mfma, use_mfma_ga, use_mfma_q6)
+    if (N >= 5 && K > 5120 && rho > 8) return false;
     return rho <= lim && K <= 8 * 4096 && (K >= 4096 || ksplit_short_rows(K));
 }
 

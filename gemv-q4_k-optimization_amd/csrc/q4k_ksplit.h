@@ -57,13 +57,8 @@ template <int V>
 __device__ __forceinline__ void ks_quantize_part(const float (&v)[V], uint32_t (&word)[V / 4], float &d8,
                                                  int &qsum, int &hsum) {
     constexpr int LPB = 32 / V;
-    bool lane_nan;
-    float amax = lane_amax(v, lane_nan);
-    if constexpr (LPB >= 2) amax = dpp_max_xor1(amax);
-    if constexpr (LPB >= 4) amax = dpp_max_xor2(amax);
-    if constexpr (LPB >= 8) amax = dpp_max_half_mirror(amax);
-    const float d = div127(amax);
-    quantize_values(v, amax, d, lane_nan, word);
+    float d;
+    quantize_lanes(v, d, word);
     int t = packed_sum(word);
     if constexpr (LPB >= 4) t += dpp<kDppXor1>(t);
     if constexpr (LPB >= 8) t += dpp<kDppXor2>(t);
@@ -447,6 +442,7 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q4k_ksplit_long_kernel(Q4K_
     static_assert(KS <= KW && (KS == KW || GMAX == 1), "short teams for rows of one partial group only");
     static_assert(!SUMS || (EPI == kEpiNone && !BATCH), "parity variants of the plain product only");
     p = with_head(p, Q4K_GEMV_HEAD_VALUES);
+    late_args(p);
     if constexpr (BATCH) batch_activation(p);
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     float *part = reinterpret_cast<float *>(lds);
@@ -558,6 +554,9 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q4k_ksplit_long_kernel(Q4K_
                 }
                 if (16 * st[k].i + SBW * slice < p.nb) {  // the wave's slice reaches this group
                     const LaneAct a = ks_read_lds(area + st[k].i * ks_slice_bytes(SBW), SBW, s, j);
+                    // read before the weights are waited for: the scheduler
+                    // put the reads below that wait, their latency after it
+                    __builtin_amdgcn_sched_barrier(0);
                     int sa, sb;
 #pragma unroll
                     for (int u = 0; u < NW; ++u) {
@@ -646,6 +645,7 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q4k_ksplit_short_nc_kernel(
     static_assert(NC >= 2 && NC <= 4 && TEAMS >= 1 && WAVES % KT == 0 && KT < KW, "short teams, 2-4 columns");
     static_assert(!RC4 || (SBW == 2 && KT == 4 && NC >= 3), "residue classes mod 4: rows of 5 to 8 blocks");
     p = with_head(p, Q4K_GEMV_HEAD_VALUES);
+    late_args(p);
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     float *part = reinterpret_cast<float *>(lds);
 

@@ -144,6 +144,15 @@ __device__ __forceinline__ GemvParams with_head(GemvParams p, const float *x, co
     return p;
 }
 
+// Named at the start of the long-row K-split kernels: arguments that are used
+// only after the quantisation.  Left to the compiler their scalar loads sink to
+// the use, behind the quantiser's rare branch or a barrier, where every wave
+// waits for them (us, MI355X: 768 x 11520 5.13 against 4.95 with them here, 1024
+// x 16384 6.57 / 6.31).
+__device__ __forceinline__ void late_args(const GemvParams &p) {
+    asm volatile("" ::"s"(p.dst), "s"(p.ld_dst), "s"(p.ring_off));
+}
+
 // Position of a wave in its sequence of (row tile, group) steps.
 struct Step {
     int tile;

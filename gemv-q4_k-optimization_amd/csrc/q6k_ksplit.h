@@ -289,6 +289,7 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q6k_ksplit_long_kernel(Q4K_
     static_assert(KS <= KW && (KS == KW || GMAX == 1), "short teams for rows of one partial group only");
     static_assert(!SUMS || (EPI == kEpiNone && !BATCH), "parity variants of the plain product only");
     p = with_head(p, Q4K_GEMV_HEAD_VALUES);
+    late_args(p);
     if constexpr (BATCH) batch_activation(p);
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     float *part = reinterpret_cast<float *>(lds);
@@ -391,6 +392,9 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q6k_ksplit_long_kernel(Q4K_
                 }
                 if (16 * st[k].i + SBW * slice < p.nb) {  // the wave's slice reaches this group
                     const Q6Act a = q6_ks_read_lds(area + st[k].i * q6_ks_slice_bytes(SBW), SBW, s, h, jp);
+                    // read before the weights are waited for: the scheduler
+                    // put the reads below that wait, their latency after it
+                    __builtin_amdgcn_sched_barrier(0);
                     int gs[4];
 #pragma unroll
                     for (int u = 0; u < NW; ++u) {
@@ -471,6 +475,7 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q6k_ksplit_short_nc_kernel(
     static_assert(NC >= 2 && NC <= 4 && TEAMS >= 1 && WAVES % KT == 0 && KT < KW, "short teams, 2-4 columns");
     static_assert(!RC4 || (SBW == 2 && KT == 4 && NC >= 3), "residue classes mod 4: rows of 5 to 8 blocks");
     p = with_head(p, Q4K_GEMV_HEAD_VALUES);
+    late_args(p);
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     float *part = reinterpret_cast<float *>(lds);
 

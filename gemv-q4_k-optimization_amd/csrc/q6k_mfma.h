@@ -53,10 +53,11 @@ namespace q4k {
 __host__ __device__ constexpr int q6m_part_bytes(int waves) { return 2 * waves * 64 * 8; }
 
 // LDS layout (bytes from the start): NC q8 columns of qcol = K + 16 bytes,
-// d8 of every 32-value block for 8 columns ([block][column], float), the
-// zero area, the partials and one weight slot per wave.
+// d8 of every 32-value block for 8 columns ([block][column], half precision,
+// as Q8_1 defines it), the zero area, the partials and one weight slot per
+// wave.
 __host__ __device__ constexpr int q6m_dk_off(int K, int nc) { return nc * mfma_qcol(K); }
-__host__ __device__ constexpr int q6m_zero_off(int K, int nc) { return q6m_dk_off(K, nc) + (K / 32) * kMfmaCols * 4; }
+__host__ __device__ constexpr int q6m_zero_off(int K, int nc) { return q6m_dk_off(K, nc) + (K / 32) * kMfmaCols * 2; }
 __host__ __device__ constexpr int q6m_part_off(int K, int nc) { return q6m_zero_off(K, nc) + kMfmaZeroBytes; }
 // Weight staging: an item (16 rows x one super-block, 16 x 210 bytes) arrives
 // with four 64-lane x 16-byte loads and goes to the wave's LDS slot, rows 224
@@ -126,14 +127,14 @@ __device__ __forceinline__ Q6MLane q6m_lane(int K, int64_t stride_col_y = 0) {
         const int c = l + 64 * i, col = c / 18, o = c - 18 * col;
         m.ya_off[i] = col < NC ? (uint32_t)(col * stride_col_y) * (uint32_t)kQ81Bytes + 16u * (uint32_t)o : kOOB;
     }
-    m.dk_off = (GA ? 0 : q6m_dk_off(K, NC)) + (2 * g) * kMfmaCols * 4;
+    m.dk_off = (GA ? 0 : q6m_dk_off(K, NC)) + (2 * g) * kMfmaCols * 2;
     return m;
 }
 
-// GA LDS layout: the d8 table ([block][8 columns], float: K bytes), a zero
+// GA LDS layout: the d8 table ([block][8 columns], half: K / 2 bytes), a zero
 // area, the partials, one weight slot and one activation slot per wave.
-__host__ __device__ constexpr int q6m_ga_zero_off(int K) { return K; }
-__host__ __device__ constexpr int q6m_ga_part_off(int K) { return K + kGaZeroBytes; }
+__host__ __device__ constexpr int q6m_ga_zero_off(int K) { return K / 2; }
+__host__ __device__ constexpr int q6m_ga_part_off(int K) { return K / 2 + kGaZeroBytes; }
 __host__ __device__ constexpr int q6m_ga_slot_off(int K, int waves) { return q6m_ga_part_off(K) + q6m_part_bytes(waves); }
 __host__ __device__ constexpr int q6m_ga_aslot_off(int K, int waves) {
     return q6m_ga_slot_off(K, waves) + waves * kQ6SlotBytes;
@@ -174,12 +175,12 @@ __device__ __forceinline__ void q6m_load(__amdgpu_buffer_rsrc_t rs, uint32_t off
 }
 
 // Writes an item to the wave's slot (GA: and its activation to the
-// activation slot); the wait and the compiler barrier keep the lanes' reads
-// of other lanes' bytes behind the writes.
+// activation slot).  The lanes read bytes other lanes wrote: a wave's LDS
+// operations execute in order, so the compiler's order is enough.
 template <bool GA = false>
 __device__ __forceinline__ void q6m_stage(uint8_t *slot, const Q6MLane &ln, const Q6MLoad &w, uint8_t *aslot = nullptr,
                                           const MfmaLoad *a = nullptr, int nc = 0) {
-    asm volatile("" ::: "memory");
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
     for (int i = 0; i < 4; ++i)
         if (i < 3 || ln.lane + 192 < kQ6Chunks) *reinterpret_cast<u32x4 *>(slot + 16 * ln.lane + 1024 * i) = w.v[i];
@@ -188,7 +189,7 @@ __device__ __forceinline__ void q6m_stage(uint8_t *slot, const Q6MLane &ln, cons
         for (int i = 0; i < 3; ++i)
             if (ln.lane + 64 * i < 18 * nc) *reinterpret_cast<u32x4 *>(aslot + 16 * (ln.lane + 64 * i)) = a->v[i];
     }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 }
 
 // 4 (w - 32) as signed bytes for four weights: ql dword (its nibble moved to
@@ -221,7 +222,7 @@ __device__ __forceinline__ void q6m_item(const GemvParams &p, const Q6MLane &ln,
     }
     const uint32_t scw = *reinterpret_cast<const uint32_t *>(wr + 192 + 4 * ln.g);
     const uint32_t dw = *reinterpret_cast<const uint32_t *>(wr + 220);  // d in the high half
-    const float *dk = reinterpret_cast<const float *>(lds + ln.dk_off + kb * (8 * kMfmaCols * 4));
+    const _Float16 *dk = reinterpret_cast<const _Float16 *>(lds + ln.dk_off + kb * (8 * kMfmaCols * 2));
     float t[kMfmaCols];
 #pragma unroll
     for (int c = 0; c < kMfmaCols; ++c) t[c] = 0.0f;
@@ -256,14 +257,13 @@ __device__ __forceinline__ void q6m_item(const GemvParams &p, const Q6MLane &ln,
         const int sc1 = __builtin_amdgcn_sbfe((int)scw, 16u * bb + 8u, 8u);
 #pragma unroll
         for (int q = 0; q < NQ; ++q) {
-            const float4 d8 = *reinterpret_cast<const float4 *>(dk + bb * kMfmaCols + 4 * q);
-            const float d8v[4] = {d8.x, d8.y, d8.z, d8.w};
+            const f16x4 d8 = *reinterpret_cast<const f16x4 *>(dk + bb * kMfmaCols + 4 * q);
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 // |4S| < 2^18 and |sc| <= 128: 24-bit products; |I| < 2^26
                 // and a multiple of 4, so exact in f32
                 const int I = __mul24(s[0][q][v], sc0) + __mul24(s[1][q][v], sc1);
-                t[4 * q + v] = __builtin_fmaf(d8v[v], (float)I, t[4 * q + v]);
+                t[4 * q + v] = __builtin_fmaf((float)d8[v], (float)I, t[4 * q + v]);
             }
         }
         if constexpr (SUMS) {
@@ -344,7 +344,7 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q6k_mfma_kernel(Q4K_GEMV_KE
     p = with_head(p, Q4K_GEMV_HEAD_VALUES);
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     int8_t *q8s = reinterpret_cast<int8_t *>(lds);
-    float *dks = reinterpret_cast<float *>(lds + q6m_dk_off(p.K, NC));
+    void *dks = lds + q6m_dk_off(p.K, NC);
 
     constexpr int kLPB = stage_lpb(NC);
     constexpr int kPreR = GA ? 1 : pre_rounds(NC, NT);
@@ -390,44 +390,34 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q6k_mfma_kernel(Q4K_GEMV_KE
     MfmaPos ahead = cur;
     Q6MLoad w[2];
     MfmaLoad av[GA ? 2 : 1];
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
+    auto issue = [&](int k) {
         q6m_load(rs, item_off(ahead), ln, w[k]);
         if constexpr (GA) q6m_load_act(ry, ln, ahead.kb, av[GA ? k : 0]);
         ahead = next(ahead);
-    }
+    };
 
     if constexpr (GA) {
-        // d8 of every (block, column); zeros for the padding columns
-        float *d8s = reinterpret_cast<float *>(lds);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) issue(k);
+        // d8 of every (block, column); the padding columns' outputs are dropped
+        uint16_t *d8s = reinterpret_cast<uint16_t *>(lds);
         for (int q = (int)threadIdx.x; q < (p.K / 32) * kMfmaCols; q += NT) {
             const int blk = q >> 3, c = q & 7;
-            float dv = 0.0f;
             if (c < NC)
-                dv = half_bits_to_float(
-                    *reinterpret_cast<const uint32_t *>(p.y + ((int64_t)c * p.stride_col_y + blk) * kQ81Bytes));
-            d8s[q] = dv;
+                d8s[q] = *reinterpret_cast<const uint16_t *>(p.y + ((int64_t)c * p.stride_col_y + blk) * kQ81Bytes);
         }
         // the zero area the A operand's zero lanes read
         if (threadIdx.x < kGaZeroBytes / 16)
             reinterpret_cast<u32x4 *>(lds + q6m_ga_zero_off(p.K))[threadIdx.x] = u32x4{0u, 0u, 0u, 0u};
     } else {
-        if (p.x)
-            stage_f32_finish<kLayoutMfmaQ6, kLPB, NT>(p.x, p.ldx, p.K, NC, p.vec_ok != 0, p.upc, xs,
-                                                      mfma_qcol(p.K), q8s, dks);
-        else
-            stage_q81_finish<kLayoutMfmaQ6, NT>(p.y, p.stride_col_y, p.K, NC, p.upc, ys, mfma_qcol(p.K), q8s,
-                                                dks);
-        // the zero area of the A operand, and d8 of the padding columns (their
-        // outputs are dropped; zeros keep them finite)
+        // the items' loads among the rounds of the quantisation, as in the
+        // Q4_K kernel
+        stage_interleaved<kLayoutMfmaQ6, kLPB, NT, 2>(p.x, p.ldx, p.y, p.stride_col_y, p.K, NC, p.vec_ok != 0, p.upc,
+                                                      xs, ys, mfma_qcol(p.K), q8s, dks, nullptr, issue);
+        // the zero area of the A operand (the padding columns' d8 stay
+        // unwritten: their outputs are dropped)
         if (threadIdx.x < kMfmaZeroBytes / 16)
             reinterpret_cast<u32x4 *>(lds + q6m_zero_off(p.K, NC))[threadIdx.x] = u32x4{0u, 0u, 0u, 0u};
-        if constexpr (NC < kMfmaCols) {
-            for (int q = (int)threadIdx.x; q < (p.K / 32) * (kMfmaCols - NC); q += NT) {
-                const int blk = q / (kMfmaCols - NC), c = NC + q - blk * (kMfmaCols - NC);
-                dks[blk * kMfmaCols + c] = 0.0f;
-            }
-        }
     }
     __syncthreads();
 
@@ -442,66 +432,64 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q6k_mfma_kernel(Q4K_GEMV_KE
                                   GA && ln.a_data[1] ? aslot + ln.ar_off[1] : lds + q6m_ga_zero_off(p.K)};
     int t = 0;                            // local segment of the current item
     int seg_end = (seg0 + 1) * p.nb >> ls;  // its end (super-block)
-    // items go two at a time (load slot k holds item it); an odd count ends
-    // with one item past the wave's, whose zeros add nothing
-    for (int it = 0; it < items;) {
+    // One item, held in load slot k; reload: then the loads of the item two
+    // further on, into the same.
+    auto item = [&](int k, bool reload) {
+        const int tile = group + ngroups * cur.r;
+        const int row = row0 + tile * kMfmaRows + ln.wrow;
+        const bool row_ok = SUMS && tile < nt && row < p.M;
+        q6m_stage<GA>(slot, ln, w[k], aslot, &av[GA ? k : 0], NC);
+        if (reload) issue(k);
+        q6m_item<NC, SUMS, GA>(p, ln, lds, slot, cur.kb, acc, row, row_ok, pa);
+        const MfmaPos done = cur;
+        cur = next(cur);
+        if (done.kb + 1 != seg_end) return;
+        float v[2];
+        q6m_segment_sums(acc, v);
+        q6m_tree_push(t, v, l1, l2, l4);
+        ++t;
+        if (t < segs) {
+            seg_end = (seg0 + t + 1) * p.nb >> ls;
+            return;
+        }
+        // round end: v is the wave's subtree of the tile
+        t = 0;
+        seg_end = (seg0 + 1) * p.nb >> ls;
+        const int buf = done.r & 1;
+        *reinterpret_cast<float2 *>(part + ((buf * WAVES + wave) * 64 + ln.lane) * 2) = make_float2(v[0], v[1]);
+        __syncthreads();
+        // outputs of this round: tile group q, column c, row rr; consecutive
+        // threads write consecutive rows of a column.  The KS subtrees
+        // combine in the same balanced tree.
+        for (int o = (int)threadIdx.x; o < ngroups * kMfmaRows * kMfmaCols; o += NT) {
+            const int rr = o & 15, c = (o >> 4) & 7, q = o >> 7;
+            const int otile = q + ngroups * done.r;
+            const int orow = row0 + otile * kMfmaRows + rr;
+            if (c < NC && otile < nt && orow < p.M) {
+                const int l64 = rr + 16 * (c >> 1);
+                const float *src = part + ((buf * WAVES + q * KS) * 64 + l64) * 2 + (c & 1);
+                float pv[kMfmaMaxSegs];
 #pragma unroll
-        for (int k = 0; k < 2; ++k, ++it) {
-            const int tile = group + ngroups * cur.r;
-            const int row = row0 + tile * kMfmaRows + ln.wrow;
-            if constexpr (GA) {
-                q6m_stage<true>(slot, ln, w[k], aslot, &av[GA ? k : 0], NC);
-                q6m_load(rs, item_off(ahead), ln, w[k]);
-                q6m_load_act(ry, ln, ahead.kb, av[GA ? k : 0]);
-                q6m_item<NC, SUMS, true>(p, ln, lds, slot, cur.kb, acc, row,
-                                         SUMS && it < items && tile < nt && row < p.M, pa);
-            } else {
-                q6m_stage(slot, ln, w[k]);
-                q6m_load(rs, item_off(ahead), ln, w[k]);
-                q6m_item<NC, SUMS>(p, ln, lds, slot, cur.kb, acc, row, SUMS && it < items && tile < nt && row < p.M,
-                                   pa);
-            }
-            ahead = next(ahead);
-            const MfmaPos done = cur;
-            cur = next(cur);
-            if (it < items && done.kb + 1 == seg_end) {
-                float v[2];
-                q6m_segment_sums(acc, v);
-                q6m_tree_push(t, v, l1, l2, l4);
-                ++t;
-                if (t < segs) {
-                    seg_end = (seg0 + t + 1) * p.nb >> ls;
-                    continue;
-                }
-                // round end: v is the wave's subtree of the tile
-                t = 0;
-                seg_end = (seg0 + 1) * p.nb >> ls;
-                const int buf = done.r & 1;
-                *reinterpret_cast<float2 *>(part + ((buf * WAVES + wave) * 64 + ln.lane) * 2) = make_float2(v[0], v[1]);
-                __syncthreads();
-                // outputs of this round: tile group q, column c, row rr;
-                // consecutive threads write consecutive rows of a column.
-                // The KS subtrees combine in the same balanced tree.
-                for (int o = (int)threadIdx.x; o < ngroups * kMfmaRows * kMfmaCols; o += NT) {
-                    const int rr = o & 15, c = (o >> 4) & 7, q = o >> 7;
-                    const int otile = q + ngroups * done.r;
-                    const int orow = row0 + otile * kMfmaRows + rr;
-                    if (c < NC && otile < nt && orow < p.M) {
-                        const int l64 = rr + 16 * (c >> 1);
-                        const float *src = part + ((buf * WAVES + q * KS) * 64 + l64) * 2 + (c & 1);
-                        float pv[kMfmaMaxSegs];
+                for (int j = 0; j < kMfmaMaxSegs; ++j) pv[j] = j < KS ? src[j * 64 * 2] : 0.0f;
 #pragma unroll
-                        for (int j = 0; j < kMfmaMaxSegs; ++j) pv[j] = j < KS ? src[j * 64 * 2] : 0.0f;
+                for (int wdt = 1; wdt < kMfmaMaxSegs; wdt *= 2)
 #pragma unroll
-                        for (int wdt = 1; wdt < kMfmaMaxSegs; wdt *= 2)
-#pragma unroll
-                            for (int j = 0; j + wdt < kMfmaMaxSegs; j += 2 * wdt)
-                                if (j + wdt < KS) pv[j] = pv[j] + pv[j + wdt];
-                        p.dst[(int64_t)c * p.ld_dst + orow] = pv[0];
-                    }
-                }
+                    for (int j = 0; j + wdt < kMfmaMaxSegs; j += 2 * wdt)
+                        if (j + wdt < KS) pv[j] = pv[j] + pv[j + wdt];
+                p.dst[(int64_t)c * p.ld_dst + orow] = pv[0];
             }
         }
+    };
+    // No loads past the wave's items, as in the Q4_K kernel.
+    int it = 0;
+    for (; it + 4 <= items; it += 2) {
+        item(0, true);
+        item(1, true);
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        if (it + k >= items) return;  // uniform; the last barrier is behind
+        item(k & 1, k == 0 && it + 2 < items);
     }
 }
 
