@@ -308,39 +308,47 @@ static bool q6_ksplit_auto(int64_t K, int64_t M, int cus, int &tr, int &waves, i
 }
 
 // Where the matrix-core kernel is chosen (all columns in one launch, which
-// the caller checks).  Measured on MI355X against the tile kernel (graph
-// replays, us):
-//  - rows of up to 4096 values: eight columns from 896 row tiles, six or more
-//    from 2048: 128256 x 4096 N=8 117.0 -> 93.5, N=6 106.7 -> 92.4;
-//    65536 x 4096 N=6 55.6 -> 49.5; 32768 x 4096 N=8 36.4 -> 29.1, N=6
-//    30.3 -> 28.5; 14336 x 4096 N=8 19.1 -> 18.3; 28672 x 3584 N=8 30.0 ->
-//    26.7.  Slower at four columns (128256 x 4096: 86.2 against 88.5), at
-//    14336 x 4096 N=6, 13824 x 3584 N=8 and on small products.
-//  - longer rows: seven or eight columns from 512 tiles (8192 x 8192 N=8
-//    24.7 -> 22.2, 8192 x 5120 N=7 19.4 -> 16.5, 28672 x 8192 N=7 53.3 ->
-//    51.9); at 5120 values also six columns from 512 tiles and five from 864
-//    (13824 x 5120 N=5 21.7 -> 21.0, 28672 x 5120 N=5 39.8 -> 33.3).  At 8192
-//    values five or six columns are slower (28672 x 8192 N=6 48.9 against
-//    51.4), and 4096 rows are slower everywhere.
-// Where the pre-quantised route runs the matrix-core kernel with its A
-// operand read from the Q8_1 buffer (GA): rows longer than 8192 values, a
-// tile per CU or more, six to eight columns, or five of rows longer than
-// 16384 values, where (the caller checks) the staged matrix-core kernel is
-// not chosen or cannot hold the columns.  Measured on MI355X (us per op
-// with a Q8_1 workspace, the quantiser launch included; GA against the tile
-// kernel): 4096 x 14336 N=8 21.88 against 24.52, N=6 20.94 / 21.59;
-// 8192 x 28672 N=8 55.79 / 89.89, N=5 52.27 / 85.27.  Even at 4096 x 14336
-// with five columns (20.75 / 20.65); slower with four (20.79 / 20.13).
-static bool use_mfma_q6_ga(int64_t M, int64_t N, int64_t K) {
-    const int64_t tiles = (M + kMfmaRows - 1) / kMfmaRows;
-    return K > 8192 && tiles >= 256 && (N >= 6 || (N == 5 && K > 16384));
-}
-
+// the caller checks); us per op on MI355X, matrix-core against the choice
+// without it, as for Q4_K (use_mfma).
+//  - rows of one or two super-blocks: three columns and more from 256 row tiles:
+//    65536 x 512 N=3 11.7 against 33.2, 8192 x 512 N=8 5.16 / 10.1.
+//  - rows of 3 to 12: five columns and more from 256 tiles, four from 9
+//    super-blocks and 1024 tiles: 32768 x 768 N=5 10.2 / 23.8, 4096 x 1536 N=6
+//    6.60 / 7.30, 4096 x 2048 N=8 6.66 / 8.57, 16384 x 2560 N=4 11.8 / 13.6, 6144
+//    x 2560 N=8 9.39 / 10.4, 4096 x 3072 N=6 7.87 / 8.44 (2048 x 768 N=6 5.94 /
+//    4.32).  Of 13: six and more (24576 x 3328 N=5 23.0 / 20.8).
+//  - rows of up to 4096: eight columns from 896 tiles, six and seven from 2048:
+//    14336 x 4096 N=8 17.3 / 19.1, 128256 x 4096 N=8 92 / 117, 32768 x 4096 N=6
+//    28.5 / 30.3 (13824 x 3584 N=8 and 14336 x 4096 N=6 are slower).
+//  - rows of up to 5120: seven and eight columns from 512 tiles, six too and
+//    five from 864 (13824 x 5120 N=5 21.0 / 21.7); of less than 8192: five and
+//    more from just over 8 rows per CU (3072 x 5376 N=8 12.5 / 15.0, 4096 x 6144
+//    N=6 11.9 / 13.3); of 8192: seven and eight from 512 tiles (8192 x 8192 N=8
+//    21.8 / 24.7; 28672 x 8192 N=6 51.4 against 48.9), five and more at 9 to 12
+//    rows per CU, where the column split ends (split_columns).
 static bool use_mfma_q6(int64_t M, int64_t N, int64_t K) {
     const int64_t tiles = (M + kMfmaRows - 1) / kMfmaRows;
+    if (K <= 512) return N >= 3 && tiles >= 256;
+    if (K <= 3328) return (N >= (K > 3072 ? 6 : 5) && tiles >= 256) || (N == 4 && K >= 2304 && K <= 3072 && tiles >= 1024);
     if (K <= 4096) return (N == 8 && tiles >= 896) || (N >= 6 && tiles >= 2048);
-    if (N >= 7 && tiles >= 512) return true;
-    return K <= 5120 && ((N == 6 && tiles >= 512) || (N == 5 && tiles >= 864));
+    if (K <= 5120) return (N >= 6 && tiles >= 512) || (N == 5 && tiles >= 864);
+    if (K < 8192) return N >= 5 && tiles > 128;
+    return (N >= 7 && tiles >= 512) || (K == 8192 && N >= 5 && tiles > 128 && tiles <= 192);
+}
+
+// Where the pre-quantised route runs the matrix-core kernel with its A
+// operand read from the Q8_1 buffer (GA): rows longer than 8192 values, five to
+// eight columns, more than 8 rows per CU (below, the column split), where (the
+// caller checks) the staged matrix-core kernel is not chosen or cannot hold
+// the columns.  Measured on MI355X (us per op with a Q8_1 workspace, the
+// quantiser launch included; GA against the tile kernel or the column split):
+// 4096 x 14336 N=8 20.9 against 24.5, N=5 20.9 / 23.4, 4096 x 11008 N=5 18.3 /
+// 19.5, 8192 x 28672 N=8 55.8 / 89.9, 3072 x 14336 N=6 20.0 / 21.8, 2432 x 9472
+// N=7 15.7 / 18.4, 2934 x 22272 N=7 27.2 / 39.9; with four columns slower (4096
+// x 14336 20.8 / 20.1), and with fewer rows (1024 x 22272 N=7 25.1 / 23.9).
+static bool use_mfma_q6_ga(int64_t M, int64_t N, int64_t K) {
+    const int64_t tiles = (M + kMfmaRows - 1) / kMfmaRows;
+    return K > 8192 && N >= 5 && tiles > 128;
 }
 
 // The matrix-core kernel's geometry, as for Q4_K: one workgroup per CU (at
@@ -362,7 +370,11 @@ static Q6Geometry pick_geometry_q6_mfma(const DeviceInfo &di, int64_t K, int64_t
     g.rows_base = (int)(tiles / g.grid);
     g.rows_extra = (int)(tiles % g.grid);
     const int64_t nt = g.rows_base + (g.rows_extra ? 1 : 0);
-    g.waves = 16;
+    // 8 waves, whose staging rounds carry the first loads of more items each
+    // (14336 x 4096 N=8 17.3 against 18.2 us, 3072 x 5376 N=8 12.4 / 13.6); 16
+    // for many tiles of rows of a full group (128256 x 4096 N=8 92.1 / 95.1,
+    // 64128 x 4096 53.9 / 54.4)
+    g.waves = tiles >= 4000 && K >= 3584 && K <= 4096 ? 16 : 8;
     if (owaves >= 1 && owaves <= 16) g.waves = owaves > 8 ? 16 : 8;
     if (ga) g.waves = 8;  // GA: its A operands in flight need more than 16 waves' registers
     const int64_t nb = K / kQK;
