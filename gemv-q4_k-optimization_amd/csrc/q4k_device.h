@@ -240,69 +240,50 @@ __host__ __device__ constexpr int group_chunk_stride(int i, int nb) {
     return 16 * (i + 1) <= nb ? 1024 : (nb & 15) * 64;
 }
 
-// LDS offset of values [4e, 4e+4) of block s (0..7) of super-block kb of
-// column c (rows of nb super-blocks), as a part of the super-block and a part
-// of the lane (chunk stride cs: group_chunk_stride in the dense layout).
+// LDS offset of values [4e, 4e+4) of 32-value block b of column c (rows of
+// nb super-blocks).
 template <int LAYOUT>
-__device__ __forceinline__ int q8_super(int c, int qcol, int kb) {
-    if (LAYOUT == kLayoutLinear || LAYOUT == kLayoutMfma || LAYOUT == kLayoutMfmaQ6) return c * qcol + kb * kQK;
-    return c * qcol + (kb >> 4) * 4096 + q4k_slot<LAYOUT>(kb & 15) * 64;
-}
-template <int LAYOUT>
-__device__ __forceinline__ int q8_lane(int s, int e, int cs = 1024) {
-    if (LAYOUT == kLayoutLinear || LAYOUT == kLayoutMfma || LAYOUT == kLayoutMfmaQ6) return s * 32 + e * 4;
+__device__ __forceinline__ int q8_offset(int c, int qcol, int nb, int b, int e) {
+    if (LAYOUT == kLayoutLinear) return c * qcol + b * 32 + e * 4;
+    const int kb = b >> 3, s = b & 7;
     if (LAYOUT == kLayoutQ4K || LAYOUT == kLayoutQ4KS2 || LAYOUT == kLayoutQ4KS4)
-        return ((s & 1) * 2 + (e >> 2)) * 1024 + (s >> 1) * 16 + (e & 3) * 4;
+        return c * qcol + (kb >> 4) * 4096 + ((s & 1) * 2 + (e >> 2)) * 1024 +
+               (q4k_slot<LAYOUT>(kb & 15) * 4 + (s >> 1)) * 16 + (e & 3) * 4;
+    const int cs = LAYOUT == kLayoutQ6KDense ? group_chunk_stride(kb >> 4, nb) : 1024;
     // Q6K: s = 4h + m, values 16j' + 4(e & 3) + [0, 4) with j' = e >> 2
-    return (s & 3) * cs + ((s >> 2) * 2 + (e >> 2)) * 16 + (e & 3) * 4;
+    return c * qcol + (kb >> 4) * 4096 + (s & 3) * cs +
+           (q4k_slot<LAYOUT>(kb & 15) * 4 + (s >> 2) * 2 + (e >> 2)) * 16 + (e & 3) * 4;
 }
 
-// The places of the auxiliary terms of block s of super-block kb of column c,
-// likewise in two parts: aux0 the d8 (in units of its type: half, float or
-// float2), aux1 the second array's (int or float units from the start of the
-// auxiliary area; half: the block's 16-value half).  total = ncols*K/32.
-template <int LAYOUT>
-__device__ __forceinline__ int aux0_super(int nblk, int c, int kb) {
-    const int pb = (nblk + 127) & ~127, at = (kb >> 4) * 16 + q4k_slot<LAYOUT>(kb & 15);  // 16i + slot
-    if (is_q6_split_layout(LAYOUT)) return c * 3 * pb + at * 8;
-    if (LAYOUT == kLayoutMfma || LAYOUT == kLayoutMfmaQ6) return kb * 64 + c;
-    if (LAYOUT == kLayoutQ4KS2 || LAYOUT == kLayoutQ4KS4) return c * pb + at * 8;
-    return c * nblk + kb * 8;
-}
-template <int LAYOUT>
-__device__ __forceinline__ int aux0_lane(int s) {
-    return LAYOUT == kLayoutMfma || LAYOUT == kLayoutMfmaQ6 ? 8 * s : s;
-}
-template <int LAYOUT>
-__device__ __forceinline__ int aux1_super(int total, int nblk, int c, int kb) {
-    const int pb = (nblk + 127) & ~127, at = (kb >> 4) * 16 + q4k_slot<LAYOUT>(kb & 15);
-    if (is_q6_split_layout(LAYOUT)) return c * 3 * pb + pb + at * 16;
-    if (is_q6_layout(LAYOUT)) return total + c * 2 * nblk + kb * 16;
-    return nblk * 4 + kb * 64 + c;  // kLayoutMfma
-}
-template <int LAYOUT>
-__device__ __forceinline__ int aux1_lane(int s, int half) {
-    if (LAYOUT == kLayoutMfma) return 8 * s;
-    return ((s >> 2) * 2 + half) * 4 + (s & 3);
+// Int index (from the start of the auxiliary area) of the Q6K offset
+// correction of half `half` of 32-value block b of column c; total = ncols*K/32.
+__device__ __forceinline__ int q6_sq_index(int total, int nblk, int c, int b, int half) {
+    const int kb = b >> 3, s = b & 7;
+    return total + c * 2 * nblk + kb * 16 + ((s >> 2) * 2 + half) * 4 + (s & 3);
 }
 
-// Stores a block's auxiliary terms at a0 = aux0, a1 = aux1 from the lane
-// holding values 16*half.. of it: d8 = half(d) widened, qsum = sum of all 32
-// q8 (Q4K/linear), hsum = sum of the lane's 16-value half (Q6K).
+// Stores the auxiliary terms of 32-value block b (qb = c*nblk + b) from the
+// lane holding values 16*half.. of it: d8 = half(d) widened, qsum = sum of
+// all 32 q8 (Q4K/linear), hsum = sum of the lane's 16-value half (Q6K).
 template <int LAYOUT>
-__device__ __forceinline__ void store_aux(void *aux, int a0, int a1, int half, float d8, int qsum, int hsum) {
-    if (is_q6_split_layout(LAYOUT) || is_q6_layout(LAYOUT)) {
-        if (half == 0) reinterpret_cast<float *>(aux)[a0] = d8;
-        reinterpret_cast<int *>(aux)[a1] = -32 * hsum;
-    } else if (LAYOUT == kLayoutMfma) {
+__device__ __forceinline__ void store_aux(void *aux, int total, int nblk, int c, int b, int qb, int half,
+                                          float d8, int qsum, int hsum) {
+    if (is_q6_split_layout(LAYOUT)) {
+        const int kb = b >> 3, s = b & 7, pb = (nblk + 127) & ~127;
+        const int at = (kb >> 4) * 16 + q4k_slot<LAYOUT>(kb & 15);  // 16i + slot
+        if (half == 0) reinterpret_cast<float *>(aux)[c * 3 * pb + at * 8 + s] = d8;
+        reinterpret_cast<int *>(aux)[c * 3 * pb + pb + at * 16 + ((s >> 2) * 2 + half) * 4 + (s & 3)] = -32 * hsum;
+    } else if (is_q6_layout(LAYOUT)) {
+        if (half == 0) reinterpret_cast<float *>(aux)[qb] = d8;
+        reinterpret_cast<int *>(aux)[q6_sq_index(total, nblk, c, b, half)] = -32 * hsum;
+    } else if (LAYOUT == kLayoutQ4KS2 || LAYOUT == kLayoutQ4KS4) {
         if (half == 0) {
-            reinterpret_cast<_Float16 *>(aux)[a0] = (_Float16)d8;
-            reinterpret_cast<float *>(aux)[a1] = d8 * (float)qsum;
+            const int kb = b >> 3, pb = (nblk + 127) & ~127;
+            reinterpret_cast<float2 *>(aux)[c * pb + (kb >> 4) * 128 + q4k_slot<LAYOUT>(kb & 15) * 8 + (b & 7)] =
+                make_float2(d8, d8 * (float)qsum);
         }
-    } else if (LAYOUT == kLayoutMfmaQ6) {
-        if (half == 0) reinterpret_cast<_Float16 *>(aux)[a0] = (_Float16)d8;
     } else if (half == 0) {
-        reinterpret_cast<float2 *>(aux)[a0] = make_float2(d8, d8 * (float)qsum);
+        reinterpret_cast<float2 *>(aux)[qb] = make_float2(d8, d8 * (float)qsum);
     }
 }
 
@@ -452,9 +433,9 @@ __device__ __forceinline__ float lane_amax(const float (&v)[V]) {
 // (2^-24): v / d lies between v r0 and v r1, and so does its rounded value.
 // One fma for each bound adds 1.5 * 2^23, which rounds to the integer (ties to
 // even) and leaves it in the low mantissa bits: where the two agree no
-// half-integer lies between the bounds (or on one: they would differ, or v is
-// 0) and the low byte is the answer (a q8 in [-127, 127] is the sum's low
-// byte).  So a value takes two fmas, one bit operation that collects the
+// half-integer lies between the bounds (one may be the lower or the upper
+// bound itself; the quotient lies strictly inside) and the low byte is the
+// answer (a q8 in [-127, 127] is the sum's low byte).  So a value takes two fmas, one bit operation that collects the
 // differences (a chain per dword) and 3/4 of a byte permute.  A block of zeros
 // passes: 0 * inf is the default NaN, low byte 0.  Where a lane of the wave has
 // a value whose bounds differ (one value in ~4 * 10^4), a NaN, or an amax so
@@ -519,119 +500,24 @@ __device__ __forceinline__ void block_sums(int v, int &half, int &full) {
     full = v;
 }
 
-// The super-blocks that a staging round of a wave covers: a unit of SPW = 8 /
-// LPB super-blocks of one column (kb and kb + 1 with kb even where SPW is 2:
-// the wave's lanes below 32 take the first, the others the second, which a
-// column with an odd number lacks in its last unit).  The units of all
-// columns in order are dealt to the workgroup's waves, round by round.  So
-// what depends on the super-block (column, address, LDS places) is
-// wave-uniform and computed on the scalar unit, and the lanes add constants:
-// each vector instruction before the first load costs a 16-wave workgroup 16
-// cycles per SIMD, and with a division and three products per lane and round
-// the loads of 14336 x 4096 N=8 were queued only 2.4 us after the start.
-// With several columns the workgroups of an XCD (blockIdx % 8) start at
-// different units: all of them read the whole activation, and in one order
-// all would wait for the first fetch of the same lines.
-template <int LPB, int NT>
-struct StageMap {
-    static constexpr int kSPW = 8 / LPB;
-    static constexpr bool kRotate = kSPW == 2;
-    static constexpr int kWaves = NT / kWave;
-    int wave, upc, units, rot, nb;
-    int e, s;        // lane: part of its block, block of its super-block
-    int second;      // lane: 1 in the unit's second super-block
-};
-
-// One round: the unit's column and (first) super-block.
-struct StagePlace {
-    int c, kb;
-    bool half;       // the unit has no second super-block
-};
-
-// Units per column of K values at LPB 4: what FastDiv arguments divide by.
-__host__ __device__ constexpr int stage_units(int K) { return (K / kQK + 1) / 2; }
-
-template <int LPB, int NT>
-__device__ __forceinline__ StageMap<LPB, NT> stage_map(int K, int ncols) {
-    typedef StageMap<LPB, NT> Map;
-    Map m;
-    m.wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    m.nb = K / kQK;
-    m.upc = Map::kSPW == 2 ? stage_units(K) : m.nb;
-    m.units = ncols * m.upc;
-    m.rot = Map::kRotate ? (int)(((blockIdx.x >> 3) & 31u) * (uint32_t)m.units >> 5) : 0;
-    const int lane = threadIdx.x & (kWave - 1);
-    m.e = lane & (LPB - 1);
-    m.s = (lane / LPB) & 7;
-    m.second = Map::kSPW == 2 ? lane >> 5 : 0;
-    return m;
-}
-
-// The wave has a round j.
-template <int LPB, int NT>
-__device__ __forceinline__ bool stage_has(const StageMap<LPB, NT> &m, int j) {
-    return m.wave + j * m.kWaves < m.units;
-}
-
-// The place of the wave's round j (a round past the last: the last).
-template <int LPB, int NT>
-__device__ __forceinline__ StagePlace stage_place(const StageMap<LPB, NT> &m, int j, int ncols, const FastDiv &fd) {
-    typedef StageMap<LPB, NT> Map;
-    int u = min(m.wave + j * Map::kWaves, m.units - 1);
-    if (Map::kRotate) {
-        u += m.rot;
-        if (u >= m.units) u -= m.units;
-    }
-    StagePlace p;
-    p.c = ncols == 1 ? 0 : (int)fastdiv((uint32_t)u, fd);
-    p.kb = Map::kSPW * (u - p.c * m.upc);
-    p.half = Map::kSPW == 2 && p.kb + 1 == m.nb;
-    return p;
-}
-
-// Where a lane's part of a round goes in LDS.
-struct StageDst {
-    int q8;          // byte offset of its values
-    int a0, a1;      // its auxiliary terms (store_aux)
-    int qb;          // the block's index c*K/32 + b
-};
-
-template <int LAYOUT, int LPB, int NT>
-__device__ __forceinline__ StageDst stage_dst(const StageMap<LPB, NT> &m, const StagePlace &p, int qcol, int ncols,
-                                              int e4, int half) {
-    const int nblk = m.nb * 8, total = ncols * nblk;
-    const int cs = LAYOUT == kLayoutQ6KDense ? group_chunk_stride(p.kb >> 4, m.nb) : 1024;
-    // the second super-block lies a constant further (kb is even)
-    StageDst d;
-    d.q8 = __builtin_amdgcn_readfirstlane(q8_super<LAYOUT>(p.c, qcol, p.kb)) +
-           (q8_lane<LAYOUT>(m.s, e4, cs) + m.second * (q8_super<LAYOUT>(0, 0, 1) - q8_super<LAYOUT>(0, 0, 0)));
-    d.a0 = __builtin_amdgcn_readfirstlane(aux0_super<LAYOUT>(nblk, p.c, p.kb)) +
-           (aux0_lane<LAYOUT>(m.s) + m.second * (aux0_super<LAYOUT>(0, 0, 1) - aux0_super<LAYOUT>(0, 0, 0)));
-    d.a1 = __builtin_amdgcn_readfirstlane(aux1_super<LAYOUT>(total, nblk, p.c, p.kb)) +
-           (aux1_lane<LAYOUT>(m.s, half) + m.second * (aux1_super<LAYOUT>(0, 0, 0, 1) - aux1_super<LAYOUT>(0, 0, 0, 0)));
-    d.qb = p.c * nblk + p.kb * 8 + (m.s + 8 * m.second);
-    return d;
-}
-
 // sq_out (parity variants only; a literal null in the product kernels, so the
 // store compiles away): the int32 sum of the block's 32 q8 at sq_out[qb].
-// live: the lane has a block (only the stores are left out without one).
 template <int LAYOUT, int LPB>
-__device__ __forceinline__ void quantize_block_part(const float (&v)[32 / LPB], int e, bool live, const StageDst &at,
-                                                    int8_t *q8s, void *aux, int32_t *sq_out = nullptr) {
+__device__ __forceinline__ void quantize_block_part(const float (&v)[32 / LPB], int e, int qcol, int c,
+                                                    int b, int qb, int total, int nblk, int8_t *q8s,
+                                                    void *aux, int32_t *sq_out = nullptr) {
     constexpr int V = 32 / LPB;
     float d;
     uint32_t word[V / 4];
     quantize_lanes(v, d, word);
     int hsum, fsum;
     block_sums<LPB>(packed_sum(word), hsum, fsum);
-    if (!live) return;
-    int8_t *dst = q8s + at.q8;
+    int8_t *dst = q8s + q8_offset<LAYOUT>(c, qcol, nblk >> 3, b, e * (V / 4));
     if (V == 4) *reinterpret_cast<uint32_t *>(dst) = word[0];
     else *reinterpret_cast<uint2 *>(dst) = make_uint2(word[0], word[V / 4 - 1]);
     const float d8 = (float)(_Float16)d;
-    if ((e & (LPB / 2 - 1)) == 0) store_aux<LAYOUT>(aux, at.a0, at.a1, e / (LPB / 2), d8, fsum, hsum);
-    if (sq_out && e == 0) sq_out[at.qb] = fsum;
+    if ((e & (LPB / 2 - 1)) == 0) store_aux<LAYOUT>(aux, total, nblk, c, b, qb, e / (LPB / 2), d8, fsum, hsum);
+    if (sq_out && e == 0) sq_out[qb] = fsum;
 }
 
 template <int V>
@@ -651,85 +537,22 @@ __device__ __forceinline__ void load_xv(const float *src, bool vec_ok, float (&v
 // NT: threads per workgroup, a compile-time constant of every kernel (reading
 // blockDim would put a dependent kernel-argument load ahead of the first
 // activation load).
-// The lane's values of a round; lanes without a super-block re-read the
-// unit's first.
-template <int LPB, int NT>
-__device__ __forceinline__ const float *stage_src(const StageMap<LPB, NT> &m, const StagePlace &p, const float *x,
-                                                  int64_t ldx) {
-    const uint32_t lane = (uint32_t)(m.s * 32 + m.e * (32 / LPB));
-    return x + (p.c * ldx + p.kb * kQK) + (p.half ? lane : lane + (uint32_t)m.second * kQK);
-}
-
 template <int LPB, int NT, int PRE>
 __device__ __forceinline__ void stage_f32_issue(const float *__restrict__ x, int64_t ldx, int K,
                                                 int ncols, bool vec_ok, const FastDiv &fd,
                                                 ActStage<LPB, PRE> &st) {
-    const auto m = stage_map<LPB, NT>(K, ncols);
+    constexpr int V = 32 / LPB;
+    const int nblk = K / 32;
+    const int total = ncols * nblk;
+    const int e = threadIdx.x & (LPB - 1);
+    constexpr int step = NT / LPB;
 #pragma unroll
     for (int j = 0; j < PRE; ++j) {
-        if (j >= 4 && j * m.kWaves >= m.units) break;  // uniform: rounds past the values are not loaded
-        load_xv<32 / LPB>(stage_src(m, stage_place(m, j, ncols, fd), x, ldx), vec_ok, st.v[j]);
-    }
-}
-
-// Values that were loaded and are not needed: the compiler waits for their
-// loads here (they are older than any weight's) and not, by waiting for
-// everything, where it next uses their registers.
-template <typename T, int V>
-__device__ __forceinline__ void stage_use(const T (&v)[V]) {
-#pragma unroll
-    for (int k = 0; k < V; ++k) asm volatile("" ::"v"(v[k]));
-}
-
-// Every load has arrived (the wave's newest were just used): tells the
-// compiler, which merges the paths with and without further rounds.
-__device__ __forceinline__ void stage_loads_done() { __builtin_amdgcn_s_waitcnt(0x0f70); }  // vmcnt(0) alone
-
-// Quantises the wave's round j, values v (nothing when it has none).
-template <int LAYOUT, int LPB, int NT>
-__device__ __forceinline__ void stage_f32_round(const StageMap<LPB, NT> &m, int j, const float (&v)[32 / LPB],
-                                                int ncols, const FastDiv &fd, int qcol, int8_t *q8s, void *aux,
-                                                int32_t *sq_out) {
-    if (!stage_has(m, j)) {  // uniform
-        stage_use(v);
-        return;
-    }
-    const StagePlace p = stage_place(m, j, ncols, fd);
-    quantize_block_part<LAYOUT, LPB>(v, m.e, !(p.half && m.second),
-                                     stage_dst<LAYOUT>(m, p, qcol, ncols, m.e * (8 / LPB), m.e / (LPB / 2)), q8s, aux,
-                                     sq_out);
-}
-
-// Rounds [j0, j1) of those in registers.
-template <int LAYOUT, int LPB, int NT, int PRE>
-__device__ __forceinline__ void stage_f32_span(const StageMap<LPB, NT> &m, int j0, int j1,
-                                               const ActStage<LPB, PRE> &st, int ncols, const FastDiv &fd, int qcol,
-                                               int8_t *q8s, void *aux, int32_t *sq_out) {
-#pragma unroll
-    for (int j = j0; j < j1; ++j) stage_f32_round<LAYOUT>(m, j, st.v[j], ncols, fd, qcol, q8s, aux, sq_out);
-}
-
-// The rounds from PRE on.
-template <int LAYOUT, int LPB, int NT, int CHUNK, int PRE>
-__device__ __forceinline__ void stage_f32_rest(const StageMap<LPB, NT> &m, const float *__restrict__ x, int64_t ldx,
-                                               int ncols, bool vec_ok, const FastDiv &fd, int qcol, int8_t *q8s,
-                                               void *aux, int32_t *sq_out) {
-    constexpr int V = 32 / LPB;
-    // A chunk of rounds at a time: all their loads first, then their
-    // quantisation, so a chunk costs one memory round trip rather than one
-    // per round.
-    constexpr int kChunk = CHUNK;
-    for (int j0 = PRE; stage_has(m, j0); j0 += kChunk) {
-        float v[kChunk][V];
-#pragma unroll
-        for (int j = 0; j < kChunk; ++j) {
-            if (j > 0 && !stage_has(m, j0 + j)) break;
-            load_xv<V>(stage_src(m, stage_place(m, j0 + j, ncols, fd), x, ldx), vec_ok, v[j]);
-        }
-#pragma unroll
-        for (int j = 0; j < kChunk; ++j)
-            stage_f32_round<LAYOUT>(m, j0 + j, v[j], ncols, fd, qcol, q8s, aux, sq_out);
-        stage_loads_done();
+        if (j >= 4 && j * step >= total) break;  // uniform: rounds past the values are not loaded
+        const int qb = min((int)(threadIdx.x / LPB) + j * step, total - 1);
+        const int c = ncols == 1 ? 0 : (int)fastdiv((uint32_t)qb, fd);
+        const int b = qb - c * nblk;
+        load_xv<V>(x + c * ldx + b * 32 + e * V, vec_ok, st.v[j]);
     }
 }
 
@@ -738,9 +561,46 @@ __device__ __forceinline__ void stage_f32_finish(const float *__restrict__ x, in
                                                  int ncols, bool vec_ok, const FastDiv &fd,
                                                  const ActStage<LPB, PRE> &st, int qcol, int8_t *q8s,
                                                  void *aux, int32_t *sq_out = nullptr) {
-    const auto m = stage_map<LPB, NT>(K, ncols);
-    stage_f32_span<LAYOUT>(m, 0, PRE, st, ncols, fd, qcol, q8s, aux, sq_out);
-    stage_f32_rest<LAYOUT, LPB, NT, CHUNK, PRE>(m, x, ldx, ncols, vec_ok, fd, qcol, q8s, aux, sq_out);
+    constexpr int V = 32 / LPB;
+    const int nblk = K / 32;
+    const int total = ncols * nblk;
+    const int e = threadIdx.x & (LPB - 1);
+    constexpr int step = NT / LPB;
+#pragma unroll
+    for (int j = 0; j < PRE; ++j) {
+        const int qb = (int)(threadIdx.x / LPB) + j * step;
+        if (qb < total) {
+            const int c = ncols == 1 ? 0 : (int)fastdiv((uint32_t)qb, fd);
+            quantize_block_part<LAYOUT, LPB>(st.v[j], e, qcol, c, qb - c * nblk, qb, total, nblk, q8s, aux,
+                                             sq_out);
+        }
+    }
+    // Further rounds a chunk at a time: all their loads first, then their
+    // quantisation, so a chunk costs one memory round trip rather than one
+    // per round.  A round past every block of the wave's lanes is not
+    // loaded (q0w, the wave's first active lane, holds its smallest block);
+    // in the others, lanes past the end re-read the last block.
+    constexpr int kChunk = CHUNK;
+    for (int q0 = (int)(threadIdx.x / LPB) + PRE * step; q0 < total; q0 += kChunk * step) {
+        const int q0w = __builtin_amdgcn_readfirstlane(q0);
+        float v[kChunk][V];
+#pragma unroll
+        for (int j = 0; j < kChunk; ++j) {
+            if (j > 0 && q0w + j * step >= total) break;
+            const int qb = min(q0 + j * step, total - 1);
+            const int c = ncols == 1 ? 0 : (int)fastdiv((uint32_t)qb, fd);
+            load_xv<V>(x + c * ldx + (qb - c * nblk) * 32 + e * V, vec_ok, v[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < kChunk; ++j) {
+            const int qb = q0 + j * step;
+            if (qb < total) {
+                const int c = ncols == 1 ? 0 : (int)fastdiv((uint32_t)qb, fd);
+                quantize_block_part<LAYOUT, LPB>(v[j], e, qcol, c, qb - c * nblk, qb, total, nblk, q8s, aux,
+                                                 sq_out);
+            }
+        }
+    }
 }
 
 // Rounds [J0, J1) of stage_f32_finish (J1 <= PRE: values already in
@@ -751,8 +611,19 @@ template <int LAYOUT, int LPB, int NT, int J0, int J1, int PRE>
 __device__ __forceinline__ void stage_f32_rounds(int K, int ncols, const FastDiv &fd, const ActStage<LPB, PRE> &st,
                                                  int qcol, int8_t *q8s, void *aux, int32_t *sq_out = nullptr) {
     static_assert(0 <= J0 && J0 <= J1 && J1 <= PRE, "rounds held in registers");
-    const auto m = stage_map<LPB, NT>(K, ncols);
-    stage_f32_span<LAYOUT>(m, J0, J1, st, ncols, fd, qcol, q8s, aux, sq_out);
+    const int nblk = K / 32;
+    const int total = ncols * nblk;
+    const int e = threadIdx.x & (LPB - 1);
+    constexpr int step = NT / LPB;
+#pragma unroll
+    for (int j = J0; j < J1; ++j) {
+        const int qb = (int)(threadIdx.x / LPB) + j * step;
+        if (qb < total) {
+            const int c = ncols == 1 ? 0 : (int)fastdiv((uint32_t)qb, fd);
+            quantize_block_part<LAYOUT, LPB>(st.v[j], e, qcol, c, qb - c * nblk, qb, total, nblk, q8s, aux,
+                                             sq_out);
+        }
+    }
 }
 
 // Already-quantised AoS block_q8_1 (column stride stride_col_y blocks) -> LDS,
@@ -763,76 +634,37 @@ struct Q81Stage {
     uint32_t ds[PRE];
 };
 
-// The lane's 8 of a block's 32 q8 and the block's ds.
-template <int NT>
-__device__ __forceinline__ void load_q81(const StageMap<4, NT> &m, const StagePlace &p,
-                                         const uint8_t *__restrict__ y, int64_t stride_col_y, uint32_t (&w)[2],
-                                         uint32_t &ds) {
-    const uint32_t lane = (uint32_t)(m.s * kQ81Bytes);
-    const uint8_t *blk = y + (p.c * stride_col_y + p.kb * 8) * kQ81Bytes +
-                         (p.half ? lane : lane + (uint32_t)(m.second * 8 * kQ81Bytes));
-    w[0] = *reinterpret_cast<const uint32_t *>(blk + 4 + m.e * 8);
-    w[1] = *reinterpret_cast<const uint32_t *>(blk + 8 + m.e * 8);
-    ds = *reinterpret_cast<const uint32_t *>(blk);
-}
-
 template <int NT, int PRE>
 __device__ __forceinline__ void stage_q81_issue(const uint8_t *__restrict__ y, int64_t stride_col_y,
                                                 int K, int ncols, const FastDiv &fd, Q81Stage<PRE> &st) {
-    const auto m = stage_map<4, NT>(K, ncols);
+    const int nblk = K / 32;
+    const int total = ncols * nblk;
+    const int quarter = threadIdx.x & 3;
+    constexpr int step = NT / 4;
 #pragma unroll
     for (int j = 0; j < PRE; ++j) {
-        if (j >= 4 && j * m.kWaves >= m.units) break;  // uniform, as above
-        load_q81(m, stage_place(m, j, ncols, fd), y, stride_col_y, st.w[j], st.ds[j]);  // unconditional, as above
+        if (j >= 4 && j * step >= total) break;  // uniform, as above
+        const int qb = min((int)(threadIdx.x >> 2) + j * step, total - 1);  // unconditional, as above
+        const int c = (int)fastdiv((uint32_t)qb, fd);
+        const uint8_t *blk = y + ((int64_t)c * stride_col_y + (qb - c * nblk)) * kQ81Bytes;
+        st.w[j][0] = *reinterpret_cast<const uint32_t *>(blk + 4 + quarter * 8);
+        st.w[j][1] = *reinterpret_cast<const uint32_t *>(blk + 8 + quarter * 8);
+        st.ds[j] = *reinterpret_cast<const uint32_t *>(blk);
     }
 }
 
 template <int LAYOUT>
-__device__ __forceinline__ void store_q81_part(uint32_t w0, uint32_t w1, uint32_t ds, int quarter, bool live,
-                                               const StageDst &at, int8_t *q8s, void *aux,
-                                               int32_t *sq_out = nullptr) {
+__device__ __forceinline__ void store_q81_part(uint32_t w0, uint32_t w1, uint32_t ds, int quarter,
+                                               int qcol, int c, int b, int qb, int total, int nblk,
+                                               int8_t *q8s, void *aux, int32_t *sq_out = nullptr) {
     int hsum, fsum;
     block_sums<4>(__builtin_amdgcn_sdot4((int)w0, 0x01010101, __builtin_amdgcn_sdot4((int)w1, 0x01010101, 0, false),
                                          false),
                   hsum, fsum);
-    if (!live) return;
-    *reinterpret_cast<uint2 *>(q8s + at.q8) = make_uint2(w0, w1);
-    if ((quarter & 1) == 0) store_aux<LAYOUT>(aux, at.a0, at.a1, quarter >> 1, half_bits_to_float(ds), fsum, hsum);
-    if (sq_out && quarter == 0) sq_out[at.qb] = fsum;
-}
-
-template <int LAYOUT, int NT>
-__device__ __forceinline__ void stage_q81_round(const StageMap<4, NT> &m, int j, const uint32_t (&w)[2], uint32_t ds,
-                                                int ncols, const FastDiv &fd, int qcol, int8_t *q8s, void *aux,
-                                                int32_t *sq_out) {
-    if (!stage_has(m, j)) {  // uniform
-        stage_use(w);
-        asm volatile("" ::"v"(ds));
-        return;
-    }
-    const StagePlace p = stage_place(m, j, ncols, fd);
-    store_q81_part<LAYOUT>(w[0], w[1], ds, m.e, !(p.half && m.second),
-                           stage_dst<LAYOUT>(m, p, qcol, ncols, 2 * m.e, m.e >> 1), q8s, aux, sq_out);
-}
-
-template <int LAYOUT, int NT, int CHUNK, int PRE>
-__device__ __forceinline__ void stage_q81_rest(const StageMap<4, NT> &m, const uint8_t *__restrict__ y,
-                                               int64_t stride_col_y, int ncols, const FastDiv &fd, int qcol,
-                                               int8_t *q8s, void *aux, int32_t *sq_out) {
-    // CHUNK rounds at a time, loads first, as in stage_f32_rest
-    constexpr int kChunk = CHUNK;
-    for (int j0 = PRE; stage_has(m, j0); j0 += kChunk) {
-        uint32_t w[kChunk][2], ds[kChunk];
-#pragma unroll
-        for (int j = 0; j < kChunk; ++j) {
-            if (j > 0 && !stage_has(m, j0 + j)) break;
-            load_q81(m, stage_place(m, j0 + j, ncols, fd), y, stride_col_y, w[j], ds[j]);
-        }
-#pragma unroll
-        for (int j = 0; j < kChunk; ++j)
-            stage_q81_round<LAYOUT>(m, j0 + j, w[j], ds[j], ncols, fd, qcol, q8s, aux, sq_out);
-        stage_loads_done();
-    }
+    *reinterpret_cast<uint2 *>(q8s + q8_offset<LAYOUT>(c, qcol, nblk >> 3, b, 2 * quarter)) = make_uint2(w0, w1);
+    if ((quarter & 1) == 0)
+        store_aux<LAYOUT>(aux, total, nblk, c, b, qb, quarter >> 1, half_bits_to_float(ds), fsum, hsum);
+    if (sq_out && quarter == 0) sq_out[qb] = fsum;
 }
 
 template <int LAYOUT, int NT, int CHUNK = kFinishRounds, int PRE>
@@ -840,40 +672,43 @@ __device__ __forceinline__ void stage_q81_finish(const uint8_t *__restrict__ y, 
                                                  int K, int ncols, const FastDiv &fd,
                                                  const Q81Stage<PRE> &st, int qcol, int8_t *q8s,
                                                  void *aux, int32_t *sq_out = nullptr) {
-    const auto m = stage_map<4, NT>(K, ncols);
+    const int nblk = K / 32;
+    const int total = ncols * nblk;
+    const int quarter = threadIdx.x & 3;
+    constexpr int step = NT / 4;
 #pragma unroll
-    for (int j = 0; j < PRE; ++j)
-        stage_q81_round<LAYOUT>(m, j, st.w[j], st.ds[j], ncols, fd, qcol, q8s, aux, sq_out);
-    stage_q81_rest<LAYOUT, NT, CHUNK, PRE>(m, y, stride_col_y, ncols, fd, qcol, q8s, aux, sq_out);
-}
-
-// stage_f32_finish or stage_q81_finish (x null: the Q8_1 columns) with N
-// other steps among its rounds: issue(k) before the k-th N-th of the rounds
-// in registers.
-template <int LAYOUT, int LPB, int NT, int N, int PRE, typename F>
-__device__ __forceinline__ void stage_interleaved(const float *__restrict__ x, int64_t ldx,
-                                                  const uint8_t *__restrict__ y, int64_t stride_col_y, int K,
-                                                  int ncols, bool vec_ok, const FastDiv &fd,
-                                                  const ActStage<LPB, PRE> &xs, const Q81Stage<PRE> &ys, int qcol,
-                                                  int8_t *q8s, void *aux, int32_t *sq_out, F issue) {
-    if (x) {
-        const auto m = stage_map<LPB, NT>(K, ncols);
-#pragma unroll
-        for (int k = 0; k < N; ++k) {
-            issue(k);
-            stage_f32_span<LAYOUT>(m, k * PRE / N, (k + 1) * PRE / N, xs, ncols, fd, qcol, q8s, aux, sq_out);
+    for (int j = 0; j < PRE; ++j) {
+        const int qb = (threadIdx.x >> 2) + j * step;
+        if (qb < total) {
+            const int c = (int)fastdiv((uint32_t)qb, fd);
+            store_q81_part<LAYOUT>(st.w[j][0], st.w[j][1], st.ds[j], quarter, qcol, c, qb - c * nblk, qb,
+                                   total, nblk, q8s, aux, sq_out);
         }
-        stage_f32_rest<LAYOUT, LPB, NT, kFinishRounds, PRE>(m, x, ldx, ncols, vec_ok, fd, qcol, q8s, aux, sq_out);
-    } else {
-        const auto m = stage_map<4, NT>(K, ncols);
+    }
+    // further rounds CHUNK at a time, loads first, as in stage_f32_finish
+    constexpr int kChunk = CHUNK;
+    for (int q0 = (threadIdx.x >> 2) + PRE * step; q0 < total; q0 += kChunk * step) {
+        const int q0w = __builtin_amdgcn_readfirstlane(q0);
+        uint32_t w[kChunk][2], ds[kChunk];
 #pragma unroll
-        for (int k = 0; k < N; ++k) {
-            issue(k);
-#pragma unroll
-            for (int j = k * PRE / N; j < (k + 1) * PRE / N; ++j)
-                stage_q81_round<LAYOUT>(m, j, ys.w[j], ys.ds[j], ncols, fd, qcol, q8s, aux, sq_out);
+        for (int j = 0; j < kChunk; ++j) {
+            if (j > 0 && q0w + j * step >= total) break;
+            const int qb = min(q0 + j * step, total - 1);
+            const int c = (int)fastdiv((uint32_t)qb, fd);
+            const uint8_t *blk = y + ((int64_t)c * stride_col_y + (qb - c * nblk)) * kQ81Bytes;
+            w[j][0] = *reinterpret_cast<const uint32_t *>(blk + 4 + quarter * 8);
+            w[j][1] = *reinterpret_cast<const uint32_t *>(blk + 8 + quarter * 8);
+            ds[j] = *reinterpret_cast<const uint32_t *>(blk);
         }
-        stage_q81_rest<LAYOUT, NT, kFinishRounds, PRE>(m, y, stride_col_y, ncols, fd, qcol, q8s, aux, sq_out);
+#pragma unroll
+        for (int j = 0; j < kChunk; ++j) {
+            const int qb = q0 + j * step;
+            if (qb < total) {
+                const int c = (int)fastdiv((uint32_t)qb, fd);
+                store_q81_part<LAYOUT>(w[j][0], w[j][1], ds[j], quarter, qcol, c, qb - c * nblk, qb, total, nblk,
+                                       q8s, aux, sq_out);
+            }
+        }
     }
 }
 

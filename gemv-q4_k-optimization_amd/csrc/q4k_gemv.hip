@@ -79,7 +79,7 @@ struct SumsParams {
     int32_t *sqq;      // [M][K/32] for this column
     int32_t *sq;       // [K/32] for this column
     int M, K, nb, G, qcol;
-    FastDiv upc;
+    FastDiv stage_div;
 };
 
 // One wave per (row, group): the GEMV's lane map, swizzled activation layout,
@@ -88,7 +88,7 @@ __global__ __launch_bounds__(256) void subblock_sums_kernel(SumsParams p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     int8_t *q8s = reinterpret_cast<int8_t *>(lds);
     float2 *dks = reinterpret_cast<float2 *>(lds + p.qcol);
-    stage_from_q8_1<kLayoutQ4K, 256>(p.y, 0, p.K, 1, p.upc, p.qcol, q8s, dks);
+    stage_from_q8_1<kLayoutQ4K, 256>(p.y, 0, p.K, 1, p.stage_div, p.qcol, q8s, dks);
     __syncthreads();
     GemvParams gp{};
     gp.w = p.w;
@@ -1047,8 +1047,7 @@ static Geometry pick_geometry(const DeviceInfo &di, int64_t K, int64_t M, int64_
         g.lds_launch = max_lds / 2 + 256;
     // weight loads before quantisation only when every activation load fits
     // the staging rounds issued ahead of them
-    const bool pro0_ok = (nc == 1 ? K / 32 : (int64_t)nc * stage_units((int)K) * 16) <=
-                         (int64_t)stage_capacity(stage_lpb(nc), g.waves * kWave, nc);
+    const bool pro0_ok = (int64_t)nc * (K / 32) <= (int64_t)stage_capacity(stage_lpb(nc), g.waves * kWave, nc);
     g.prologue = pro0_ok ? 0 : 1;
     // One column and two slots on streams of under 8 steps per wave: one
     // early group instead of two (measured on MI355X: 4096 x 14336 9.06 ->
@@ -1341,7 +1340,7 @@ static int run_gemv(const void *src0, int64_t ne00, int64_t ne01, int64_t nb01, 
         p.G = (p.nb + 15) / 16;
         p.qcol = q8_col_bytes((int)ne00);
         p.ntiles = geo.ntiles;
-        p.upc = fastdiv_init((uint32_t)stage_units((int)ne00));
+        p.stage_div = fastdiv_init((uint32_t)(ne00 / 32));
         if (so) {  // parity variant: each column's launch on its own, same geometry and kernel
             for (int64_t c = 0; c < ncols; ++c) {
                 GemvParams pc = p;
@@ -1399,7 +1398,7 @@ static int run_gemv(const void *src0, int64_t ne00, int64_t ne01, int64_t nb01, 
         p.qcol = q8_col_bytes((int)ne00);
         p.ntiles = geo.ntiles;
         p.vec_ok = x && aligned(p.x, 16) && (ldx % 4 == 0);
-        p.upc = fastdiv_init((uint32_t)stage_units((int)ne00));
+        p.stage_div = fastdiv_init((uint32_t)(geo.mfma ? stage_units((int)ne00) : ne00 / 32));
         if (fused) {
             p.gate = ep->gate;
             p.bias = ep->bias;
@@ -1809,7 +1808,7 @@ int q4k_subblock_sums(const void *src0, int64_t ne00, int64_t ne01, int64_t nb01
         p.nb = nb;
         p.G = (nb + 15) / 16;
         p.qcol = q8_col_bytes((int)ne00);
-        p.upc = fastdiv_init((uint32_t)stage_units((int)ne00));
+        p.stage_div = fastdiv_init((uint32_t)(ne00 / 32));
         const int64_t items = ne01 * p.G;
         int grid = (int)((items + 3) / 4);
         if (grid > di->cus * 8) grid = di->cus * 8;

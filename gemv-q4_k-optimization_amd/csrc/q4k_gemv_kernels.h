@@ -250,15 +250,6 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q4k_kernel(Q4K_GEMV_KERNEL_
     int8_t *q8s = reinterpret_cast<int8_t *>(lds);
     float2 *dks = reinterpret_cast<float2 *>(lds + NC * p.qcol);
 
-    // first of all the activation loads: everything waits for them
-    constexpr int kLPB = stage_lpb(NC);  // activation lanes per 32-value block
-    constexpr int kPreR = pre_rounds(NC, kWave * WAVES);
-    ActStage<kLPB, kPreR> xs;
-    Q81Stage<kPreR> ys;
-    if (p.x) stage_f32_issue<kLPB, kWave * WAVES>(p.x, p.ldx, p.K, NC, p.vec_ok != 0, p.upc, xs);
-    else stage_q81_issue<kWave * WAVES>(p.y, p.stride_col_y, p.K, NC, p.upc, ys);
-    __builtin_amdgcn_sched_barrier(0);
-
     Lane ln;
     ln.lane = threadIdx.x & (kWave - 1);
     ln.g = ln.lane >> 2;
@@ -269,7 +260,15 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q4k_kernel(Q4K_GEMV_KERNEL_
     // row numbers and buffer descriptors in scalar registers
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const WaveRows wr = wave_rows<WAVES>(p, wave);
-    if constexpr (BATCH) batch_weights(p);
+    constexpr int kLPB = stage_lpb(NC);  // activation lanes per 32-value block
+    constexpr int kPreR = pre_rounds(NC, kWave * WAVES);
+    ActStage<kLPB, kPreR> xs;
+    Q81Stage<kPreR> ys;
+    if constexpr (BATCH) {
+        if (p.x) stage_f32_issue<kLPB, kWave * WAVES>(p.x, p.ldx, p.K, NC, p.vec_ok != 0, p.stage_div, xs);
+        else stage_q81_issue<kWave * WAVES>(p.y, p.stride_col_y, p.K, NC, p.stage_div, ys);
+        batch_weights(p);
+    }
     const bool absent = BATCH && p.w_absent;
     const WaveStream ws = wave_stream(p, ln, wr, GLU ? 1 : R, absent);
     const __amdgpu_buffer_rsrc_t rs_gate =
@@ -278,6 +277,10 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q4k_kernel(Q4K_GEMV_KERNEL_
             : ws.rs;
     int remaining = ws.ntiles * p.G;  // steps of this wave
 
+    if constexpr (!BATCH) {
+        if (p.x) stage_f32_issue<kLPB, kWave * WAVES>(p.x, p.ldx, p.K, NC, p.vec_ok != 0, p.stage_div, xs);
+        else stage_q81_issue<kWave * WAVES>(p.y, p.stride_col_y, p.K, NC, p.stage_div, ys);
+    }
     __syncthreads();  // all activation loads of this CU are queued first
 
     Step st[S];
@@ -287,9 +290,6 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q4k_kernel(Q4K_GEMV_KERNEL_
     for (int k = 1; k < S; ++k) st[k] = next_step(st[k - 1], p.G);
 #pragma unroll
     for (int k = 0; k < kEarly; ++k) load_step<R, GLU>(p, ln, ws, rs_gate, st[k], w[k]);
-    // dst is loaded by now, not after the last barrier (4096 x 4096 N=4 6.33 ->
-    // 6.10 us)
-    asm volatile("" ::"s"(p.dst));
     float acc[R][NC];
 #pragma unroll
     for (int r = 0; r < R; ++r)
@@ -309,12 +309,12 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q4k_kernel(Q4K_GEMV_KERNEL_
     // early weights still in flight and 4096 x 14336 went 9.07 -> 9.41 us.
     constexpr bool kStream = NC == 1 && R == 1 && PRO == 0 && S == 2 && kEarly == 2 && WAVES == 16;
     if (kStream && p.x && p.G == 2) {
-        stage_f32_rounds<kLayoutQ4K, kLPB, kWave * WAVES, 0, 1>(p.K, NC, p.upc, xs, p.qcol, q8s, dks, sq_out);
+        stage_f32_rounds<kLayoutQ4K, kLPB, kWave * WAVES, 0, 1>(p.K, NC, p.stage_div, xs, p.qcol, q8s, dks, sq_out);
         __syncthreads();
         process_group<NC, R, EPI, SUMS>(p, ln, st[0], q8s, dks, w[0], acc, rr);
         st[0] = next_step(st[S - 1], p.G);
         load_step<R, GLU>(p, ln, ws, rs_gate, st[0], w[0]);
-        stage_f32_rounds<kLayoutQ4K, kLPB, kWave * WAVES, 1, 2>(p.K, NC, p.upc, xs, p.qcol, q8s, dks, sq_out);
+        stage_f32_rounds<kLayoutQ4K, kLPB, kWave * WAVES, 1, 2>(p.K, NC, p.stage_div, xs, p.qcol, q8s, dks, sq_out);
         __syncthreads();
         process_group<NC, R, EPI, SUMS>(p, ln, st[1], q8s, dks, w[1], acc, rr);
         st[1] = next_step(st[0], p.G);
@@ -327,10 +327,10 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q4k_kernel(Q4K_GEMV_KERNEL_
     } else {
         if (p.x)
             stage_f32_finish<kLayoutQ4K, kLPB, kWave * WAVES, NC < 4 ? 1 : kFinishRounds>(
-                p.x, p.ldx, p.K, NC, p.vec_ok != 0, p.upc, xs, p.qcol, q8s, dks, sq_out);
+                p.x, p.ldx, p.K, NC, p.vec_ok != 0, p.stage_div, xs, p.qcol, q8s, dks, sq_out);
         else
             stage_q81_finish<kLayoutQ4K, kWave * WAVES, NC < 4 ? 1 : kFinishRounds>(
-                p.y, p.stride_col_y, p.K, NC, p.upc, ys, p.qcol, q8s, dks, sq_out);
+                p.y, p.stride_col_y, p.K, NC, p.stage_div, ys, p.qcol, q8s, dks, sq_out);
         __syncthreads();
         if (remaining == 0) return;  // no barrier below this point
 #pragma unroll
@@ -495,17 +495,17 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q4k_bpl_kernel(Q4K_GEMV_KER
     // each wave's first two passes
     ActStage<8, pre_rounds(1, kWave * WAVES)> xs;
     Q81Stage<pre_rounds(1, kWave * WAVES)> ys;
-    if (p.x) stage_f32_issue<8, kWave * WAVES>(p.x, p.ldx, p.K, 1, p.vec_ok != 0, p.upc, xs);
-    else stage_q81_issue<kWave * WAVES>(p.y, p.stride_col_y, p.K, 1, p.upc, ys);
+    if (p.x) stage_f32_issue<8, kWave * WAVES>(p.x, p.ldx, p.K, 1, p.vec_ok != 0, p.stage_div, xs);
+    else stage_q81_issue<kWave * WAVES>(p.y, p.stride_col_y, p.K, 1, p.stage_div, ys);
     __syncthreads();
     u32x4 wa[9], wb[9];
     if (active) load_pass(p, pa, rr, kb, lane_on, wa);
     if (vb) load_pass(p, pb, rr, kb, lane_on, wb);
     if (p.x)
-        stage_f32_finish<kLayoutLinear, 8, kWave * WAVES, 1>(p.x, p.ldx, p.K, 1, p.vec_ok != 0, p.upc, xs, p.K, q8s,
+        stage_f32_finish<kLayoutLinear, 8, kWave * WAVES, 1>(p.x, p.ldx, p.K, 1, p.vec_ok != 0, p.stage_div, xs, p.K, q8s,
                                                           dks, sq_out);
     else
-        stage_q81_finish<kLayoutLinear, kWave * WAVES, 1>(p.y, p.stride_col_y, p.K, 1, p.upc, ys, p.K, q8s, dks,
+        stage_q81_finish<kLayoutLinear, kWave * WAVES, 1>(p.y, p.stride_col_y, p.K, 1, p.stage_div, ys, p.K, q8s, dks,
                                                        sq_out);
     __syncthreads();
     if (!active) return;  // no barrier below this point
@@ -621,14 +621,14 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q4k_blk_kernel(Q4K_GEMV_KER
     // each wave's first two passes
     ActStage<8, pre_rounds(1, kWave * WAVES)> xs;
     Q81Stage<pre_rounds(1, kWave * WAVES)> ys;
-    if (p.x) stage_f32_issue<8, kWave * WAVES>(p.x, p.ldx, p.K, 1, p.vec_ok != 0, p.upc, xs);
-    else stage_q81_issue<kWave * WAVES>(p.y, p.stride_col_y, p.K, 1, p.upc, ys);
+    if (p.x) stage_f32_issue<8, kWave * WAVES>(p.x, p.ldx, p.K, 1, p.vec_ok != 0, p.stage_div, xs);
+    else stage_q81_issue<kWave * WAVES>(p.y, p.stride_col_y, p.K, 1, p.stage_div, ys);
     __syncthreads();
     u32x4 wa[9], wb[9];
     if (active) load_pass_coalesced(p, pa, po, wa);
     if (vb) load_pass_coalesced(p, pb, po, wb);
-    if (p.x) stage_f32_finish<kLayoutLinear, 8, kWave * WAVES, 1>(p.x, p.ldx, p.K, 1, p.vec_ok != 0, p.upc, xs, p.K, q8s, dks);
-    else stage_q81_finish<kLayoutLinear, kWave * WAVES, 1>(p.y, p.stride_col_y, p.K, 1, p.upc, ys, p.K, q8s, dks);
+    if (p.x) stage_f32_finish<kLayoutLinear, 8, kWave * WAVES, 1>(p.x, p.ldx, p.K, 1, p.vec_ok != 0, p.stage_div, xs, p.K, q8s, dks);
+    else stage_q81_finish<kLayoutLinear, kWave * WAVES, 1>(p.y, p.stride_col_y, p.K, 1, p.stage_div, ys, p.K, q8s, dks);
     __syncthreads();
     if (!active) return;  // no barrier below this point
 

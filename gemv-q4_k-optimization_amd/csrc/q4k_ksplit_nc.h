@@ -141,7 +141,7 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q4k_ksplit_nc_kernel(Q4K_GE
     float xv[STAGED ? 1 : G][NC][V];
     ActStage<kLPB, kPreR> xs;
     if constexpr (STAGED) {
-        stage_f32_issue<kLPB, kWave * WAVES>(p.x, p.ldx, p.K, NC, true, p.upc, xs);
+        stage_f32_issue<kLPB, kWave * WAVES>(p.x, p.ldx, p.K, NC, true, p.stage_div, xs);
         __syncthreads();
     } else {
 #pragma unroll
@@ -201,7 +201,7 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q4k_ksplit_nc_kernel(Q4K_GE
         int8_t *q8s = reinterpret_cast<int8_t *>(lds);
         float2 *dks = reinterpret_cast<float2 *>(lds + NC * p.qcol);
         stage_f32_finish<kLayout, kLPB, kWave * WAVES, NC < 4 ? 1 : kFinishRounds>(
-            p.x, p.ldx, p.K, NC, true, p.upc, xs, p.qcol, q8s, dks, SUMS ? p.sq : nullptr);
+            p.x, p.ldx, p.K, NC, true, p.stage_div, xs, p.qcol, q8s, dks, SUMS ? p.sq : nullptr);
         __syncthreads();
 #pragma unroll
         for (int i = 0; i < G; ++i)
@@ -334,13 +334,6 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q4k_ksplit_nc_long_kernel(Q
     float2 *dks = reinterpret_cast<float2 *>(lds + NC * p.qcol);
     float *part = reinterpret_cast<float *>(lds + p.ring_off);
 
-    // 1. first of all the staging loads of every wave, queued ahead of the
-    //    weight loads by the barrier below
-    constexpr int kLPB = stage_lpb(NC);
-    constexpr int kPreR = pre_rounds(NC, kWave * WAVES);
-    ActStage<kLPB, kPreR> xs;
-    stage_f32_issue<kLPB, kWave * WAVES>(p.x, p.ldx, p.K, NC, true, p.upc, xs);
-    __builtin_amdgcn_sched_barrier(0);
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int slice = wave % KW, team = wave / KW;
@@ -357,6 +350,11 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q4k_ksplit_nc_long_kernel(Q
     const int kb0 = ksn_block<P, SBW>(slice, s);       // the lane's super-block within each group
     const int wkb = ksn_block<P, SBW>(slice, 0);       // the wave's first one
 
+    // 1. the staging loads of every wave, queued ahead of the weight loads
+    constexpr int kLPB = stage_lpb(NC);
+    constexpr int kPreR = pre_rounds(NC, kWave * WAVES);
+    ActStage<kLPB, kPreR> xs;
+    stage_f32_issue<kLPB, kWave * WAVES>(p.x, p.ldx, p.K, NC, true, p.stage_div, xs);
     __syncthreads();
 
     // 2. the first S steps' weights
@@ -383,7 +381,7 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q4k_ksplit_nc_long_kernel(Q
 
     // 3. quantise into LDS (the tile kernel's layout and arithmetic)
     stage_f32_finish<kLayout, kLPB, kWave * WAVES, NC < 4 ? 1 : kFinishRounds>(
-        p.x, p.ldx, p.K, NC, true, p.upc, xs, p.qcol, q8s, dks, SUMS ? p.sq : nullptr);
+        p.x, p.ldx, p.K, NC, true, p.stage_div, xs, p.qcol, q8s, dks, SUMS ? p.sq : nullptr);
     __syncthreads();
 
     const int sl = q4k_slot<kLayout>(kb0);  // its slot in the staged layout

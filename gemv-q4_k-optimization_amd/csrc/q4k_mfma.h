@@ -67,6 +67,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include "q4k_stage_units.h"
 #include "q4k_tile.h"
 
 namespace q4k {
@@ -469,8 +470,8 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q4k_mfma_kernel(Q4K_GEMV_KE
     Q81Stage<kPreR> ys;
     if constexpr (!GA) {
         // first of all: everything waits for the activation
-        if (p.x) stage_f32_issue<kLPB, NT>(p.x, p.ldx, p.K, NC, p.vec_ok != 0, p.upc, xs);
-        else stage_q81_issue<NT>(p.y, p.stride_col_y, p.K, NC, p.upc, ys);
+        if (p.x) unit_f32_issue<kLPB, NT>(p.x, p.ldx, p.K, NC, p.vec_ok != 0, p.stage_div, xs);
+        else unit_q81_issue<NT>(p.y, p.stride_col_y, p.K, NC, p.stage_div, ys);
         __builtin_amdgcn_sched_barrier(0);
     }
     MfmaLane ln = mfma_lane<NC, GA>(p.K, p.stride_col_y);
@@ -535,7 +536,7 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q4k_mfma_kernel(Q4K_GEMV_KE
         // the items' loads among the rounds of the quantisation: issued
         // together ahead of it, the waves whose requests queued last stood
         // still until most of the others' data had arrived
-        stage_interleaved<kLayoutMfma, kLPB, NT, NIF>(p.x, p.ldx, p.y, p.stride_col_y, p.K, NC, p.vec_ok != 0, p.upc,
+        stage_interleaved<kLayoutMfma, kLPB, NT, NIF>(p.x, p.ldx, p.y, p.stride_col_y, p.K, NC, p.vec_ok != 0, p.stage_div,
                                                       xs, ys, __builtin_amdgcn_readfirstlane(mfma_qcol(p.K)), q8s, aux,
                                                       sq_out, issue);
         // the zero area of the A operand (the padding columns' d8 stay

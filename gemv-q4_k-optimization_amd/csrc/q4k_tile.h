@@ -46,7 +46,7 @@ struct GemvParams {
     int rows_base;           // tile kernel: each workgroup owns rows_base rows,
     int rows_extra;          //   the first rows_extra workgroups one more
     int ring_off;            // tile kernel: LDS byte offset of the per-wave result rings
-    FastDiv upc;             // division by a column's staging units (stage_units)
+    FastDiv stage_div;       // division by K/32 (Q8_1 blocks per column); matrix-core kernels: by stage_units
     // fused epilogue (one column): gate weight rows (same layout as w), the
     // biases of the two products (indexed like dst) and the GLU op
     const uint8_t *gate;

@@ -26,14 +26,14 @@ struct Q6SumsParams {
     const uint8_t *y;  // one column of AoS Q8_1
     int32_t *s16;      // [M][K/16] for this column
     int M, K, nb, G, qcol;
-    FastDiv upc;
+    FastDiv stage_div;
 };
 
 __global__ __launch_bounds__(256) void q6_group_sums_kernel(Q6SumsParams p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     int8_t *q8s = reinterpret_cast<int8_t *>(lds);
     uint8_t *aux = lds + p.qcol;
-    stage_from_q8_1<kLayoutQ6K, 256>(p.y, 0, p.K, 1, p.upc, p.qcol, q8s, aux);
+    stage_from_q8_1<kLayoutQ6K, 256>(p.y, 0, p.K, 1, p.stage_div, p.qcol, q8s, aux);
     __syncthreads();
     GemvParams gp{};
     gp.K = p.K;
@@ -577,8 +577,7 @@ static Q6Geometry pick_geometry_q6(const DeviceInfo &di, int64_t K, int64_t M, i
     g.lds = q6_tile_lds_bytes((int)K, nc, g.waves, g.dense);
     g.lds_launch = g.lds;
     if (owgs == 0 && g.lds_launch <= max_lds / 2) g.lds_launch = max_lds / 2 + 256;
-    const bool pro0_ok = (nc == 1 ? K / 32 : (int64_t)nc * stage_units((int)K) * 16) <=
-                         (int64_t)stage_capacity(stage_lpb(nc), g.waves * kWave, nc);
+    const bool pro0_ok = (int64_t)nc * (K / 32) <= (int64_t)stage_capacity(stage_lpb(nc), g.waves * kWave, nc);
     g.prologue = pro0_ok ? 0 : 1;
     const int opro = g_ovr_prologue.load();
     if (opro == 1 || (opro == 0 && pro0_ok)) g.prologue = opro;
@@ -736,7 +735,7 @@ int run_gemv_q6(const void *src0, int64_t ne00, int64_t ne01, int64_t nb01, cons
         p.rows_base = geo.rows_base;
         p.rows_extra = geo.rows_extra;
         p.ring_off = q6_act_bytes(p.K, nc, dense);
-        p.upc = fastdiv_init((uint32_t)stage_units((int)ne00));
+        p.stage_div = fastdiv_init((uint32_t)(geo.mfma ? stage_units((int)ne00) : ne00 / 32));
         if (fused) {
             p.gate = ep->gate;
             p.bias = ep->bias;
@@ -941,7 +940,7 @@ int q6k_group_sums(const void *src0, int64_t ne00, int64_t ne01, int64_t nb01, c
         p.nb = nb;
         p.G = (nb + 15) / 16;
         p.qcol = q8_col_bytes((int)ne00);
-        p.upc = fastdiv_init((uint32_t)stage_units((int)ne00));
+        p.stage_div = fastdiv_init((uint32_t)(ne00 / 32));
         const int64_t items = ne01 * p.G;
         int grid = (int)((items + 3) / 4);
         if (grid > di->cus * 8) grid = di->cus * 8;

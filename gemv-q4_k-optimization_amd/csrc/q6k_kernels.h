@@ -298,19 +298,18 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q6k_kernel(Q4K_GEMV_KERNEL_
     int8_t *q8s = reinterpret_cast<int8_t *>(lds);
     uint8_t *aux = lds + NC * p.qcol;
 
-    // first of all the activation loads: everything waits for them
-    constexpr int kLPB = stage_lpb(NC);  // activation lanes per 32-value block
-    constexpr int kPreR = pre_rounds(NC, kWave * WAVES);
-    ActStage<kLPB, kPreR> xs;
-    Q81Stage<kPreR> ys;
-    if (p.x) stage_f32_issue<kLPB, kWave * WAVES>(p.x, p.ldx, p.K, NC, p.vec_ok != 0, p.upc, xs);
-    else stage_q81_issue<kWave * WAVES>(p.y, p.stride_col_y, p.K, NC, p.upc, ys);
-    __builtin_amdgcn_sched_barrier(0);
-
     const Q6Lane ln = q6_lane(threadIdx.x & (kWave - 1));
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const WaveRows wr = wave_rows<WAVES>(p, wave);
-    if constexpr (BATCH) batch_weights(p);
+    constexpr int kLPB = stage_lpb(NC);
+    constexpr int kPreR = pre_rounds(NC, kWave * WAVES);
+    ActStage<kLPB, kPreR> xs;
+    Q81Stage<kPreR> ys;
+    if constexpr (BATCH) {
+        if (p.x) stage_f32_issue<kLPB, kWave * WAVES>(p.x, p.ldx, p.K, NC, p.vec_ok != 0, p.stage_div, xs);
+        else stage_q81_issue<kWave * WAVES>(p.y, p.stride_col_y, p.K, NC, p.stage_div, ys);
+        batch_weights(p);
+    }
     Q6Stream ws;
     const uint32_t wave_bytes = BATCH && p.w_absent ? 0u : (uint32_t)((wr.end - wr.beg) * p.row_stride);
     ws.rs = make_rsrc(p.w + (int64_t)wr.beg * p.row_stride, wave_bytes);
@@ -318,6 +317,10 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q6k_kernel(Q4K_GEMV_KERNEL_
     ws.ntiles = wr.end - wr.beg;
     int remaining = ws.ntiles * p.G;
 
+    if constexpr (!BATCH) {
+        if (p.x) stage_f32_issue<kLPB, kWave * WAVES>(p.x, p.ldx, p.K, NC, p.vec_ok != 0, p.stage_div, xs);
+        else stage_q81_issue<kWave * WAVES>(p.y, p.stride_col_y, p.K, NC, p.stage_div, ys);
+    }
     __syncthreads();  // all activation loads of this CU are queued first
 
     Step st[S];
@@ -327,15 +330,12 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q6k_kernel(Q4K_GEMV_KERNEL_
     for (int k = 1; k < S; ++k) st[k] = next_step(st[k - 1], p.G);
 #pragma unroll
     for (int k = 0; k < kEarly; ++k) q6_load_step<R>(p, ln, ws, st[k], w[k]);
-    // dst is loaded by now, not after the last barrier (4096 x 4096 N=4 6.33 ->
-    // 6.10 us)
-    asm volatile("" ::"s"(p.dst));
     if (p.x)
         stage_f32_finish<kLayout, kLPB, kWave * WAVES, NC < 4 ? 1 : kFinishRounds>(
-            p.x, p.ldx, p.K, NC, p.vec_ok != 0, p.upc, xs, p.qcol, q8s, aux);
+            p.x, p.ldx, p.K, NC, p.vec_ok != 0, p.stage_div, xs, p.qcol, q8s, aux);
     else
         stage_q81_finish<kLayout, kWave * WAVES, NC < 4 ? 1 : kFinishRounds>(
-            p.y, p.stride_col_y, p.K, NC, p.upc, ys, p.qcol, q8s, aux);
+            p.y, p.stride_col_y, p.K, NC, p.stage_div, ys, p.qcol, q8s, aux);
     __syncthreads();
     if (remaining == 0) return;  // no barrier below this point
 #pragma unroll

@@ -99,7 +99,7 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q6k_ksplit_nc_kernel(Q4K_GE
     constexpr int kLPB = stage_lpb(NC);
     constexpr int kPreR = pre_rounds(NC, kWave * WAVES);
     ActStage<kLPB, kPreR> xs;
-    stage_f32_issue<kLPB, kWave * WAVES>(p.x, p.ldx, p.K, NC, true, p.upc, xs);
+    stage_f32_issue<kLPB, kWave * WAVES>(p.x, p.ldx, p.K, NC, true, p.stage_div, xs);
     __syncthreads();
 
     // 2. the first S steps' weights
@@ -128,7 +128,7 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q6k_ksplit_nc_kernel(Q4K_GE
     for (int k = 0; k < S; ++k) load_step(st[k], w[k]);
 
     // 3. quantise into LDS (the tile kernel's Q6_K staging arithmetic)
-    stage_f32_finish<kLayout, kLPB, kWave * WAVES, NC < 4 ? 1 : kFinishRounds>(p.x, p.ldx, p.K, NC, true, p.upc,
+    stage_f32_finish<kLayout, kLPB, kWave * WAVES, NC < 4 ? 1 : kFinishRounds>(p.x, p.ldx, p.K, NC, true, p.stage_div,
                                                                                 xs, p.qcol, q8s, aux);
     __syncthreads();
 

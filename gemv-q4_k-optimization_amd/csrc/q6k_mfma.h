@@ -352,8 +352,8 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q6k_mfma_kernel(Q4K_GEMV_KE
     Q81Stage<kPreR> ys;
     if constexpr (!GA) {
         // first of all: everything waits for the activation
-        if (p.x) stage_f32_issue<kLPB, NT>(p.x, p.ldx, p.K, NC, p.vec_ok != 0, p.upc, xs);
-        else stage_q81_issue<NT>(p.y, p.stride_col_y, p.K, NC, p.upc, ys);
+        if (p.x) unit_f32_issue<kLPB, NT>(p.x, p.ldx, p.K, NC, p.vec_ok != 0, p.stage_div, xs);
+        else unit_q81_issue<NT>(p.y, p.stride_col_y, p.K, NC, p.stage_div, ys);
         __builtin_amdgcn_sched_barrier(0);
     }
     Q6MLane ln = q6m_lane<NC, GA>(p.K, p.stride_col_y);
@@ -412,7 +412,7 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q6k_mfma_kernel(Q4K_GEMV_KE
     } else {
         // the items' loads among the rounds of the quantisation, as in the
         // Q4_K kernel
-        stage_interleaved<kLayoutMfmaQ6, kLPB, NT, 2>(p.x, p.ldx, p.y, p.stride_col_y, p.K, NC, p.vec_ok != 0, p.upc,
+        stage_interleaved<kLayoutMfmaQ6, kLPB, NT, 2>(p.x, p.ldx, p.y, p.stride_col_y, p.K, NC, p.vec_ok != 0, p.stage_div,
                                                       xs, ys, mfma_qcol(p.K), q8s, dks, nullptr, issue);
         // the zero area of the A operand (the padding columns' d8 stay
         // unwritten: their outputs are dropped)
