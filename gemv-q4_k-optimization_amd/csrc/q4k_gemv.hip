@@ -294,13 +294,18 @@ static bool use_mfma_ga(int64_t M, int64_t N, int64_t K) {
     return K > 8192 && N >= 5 && tiles > 128;
 }
 
+// Waves per workgroup of the matrix-core kernel: 8 (16 measured slower from few
+// tiles on: 14336 x 4096 N=8 14.2 against 13.6 us), or as the override says.
+static int mfma_waves(int owaves) { return owaves > 8 && owaves <= 16 ? 16 : 8; }
+
 // The matrix-core kernel: one workgroup per CU (at most one per tile) of 8
 // or 16 waves, the tiles of 16 rows split evenly over the workgroups, and as
 // many waves sharing a tile (KS) as leave every wave group a tile in the
 // first round -- KS at most the S summation segments of a row (S = min(8,
 // the largest power of two <= the super-blocks per row), a function of K
 // alone, which fixes the summation order).
-static Geometry pick_geometry_mfma(const DeviceInfo &di, int64_t K, int64_t M, int nc, int owgs, bool ga = false) {
+static Geometry pick_geometry_mfma(const DeviceInfo &di, int64_t K, int64_t M, int nc, int owgs, int owaves,
+                                   bool ga = false) {
     Geometry g;
     const int max_lds = di.max_lds > 0 ? di.max_lds : 65536;
     const int cus = di.cus > 0 ? di.cus : 1;
@@ -315,8 +320,11 @@ static Geometry pick_geometry_mfma(const DeviceInfo &di, int64_t K, int64_t M, i
     g.rows_base = (int)(tiles / g.grid);
     g.rows_extra = (int)(tiles % g.grid);
     const int64_t nt = g.rows_base + (g.rows_extra ? 1 : 0);
-    g.waves = 8;  // 16 measured slower from few tiles on (14336 x 4096 N=8 14.2 against 13.6 us)
-    if (ga) g.slots = g_ovr_slots.load() == 4 ? 4 : 2;
+    g.waves = mfma_waves(owaves);
+    if (ga) {  // (its A operands in flight need more registers than 16 waves have)
+        g.waves = 8;
+        g.slots = g_ovr_slots.load() == 4 ? 4 : 2;
+    }
     const int64_t nb = K / kQK;
     g.segs = 1;
     while (g.segs < kMfmaMaxSegs && 2 * g.segs <= nb) g.segs *= 2;
@@ -939,12 +947,12 @@ static Geometry pick_geometry(const DeviceInfo &di, int64_t K, int64_t M, int64_
     if (q81 && !fused && mats == 1 && N <= kMfmaCols &&
         (okern == 6 || (okern == 0 && use_mfma_ga(M, N, K) &&
                          !(use_mfma(M, N, K) && mfma_lds_bytes((int)K, (int)N, 16) <= max_lds))))
-        return pick_geometry_mfma(di, K, M, (int)N, owgs, true);
+        return pick_geometry_mfma(di, K, M, (int)N, owgs, owaves, true);
     if (!fused && mats == 1 && (okern == 4 || (okern == 0 && use_mfma(M, N, K)))) {
         int mc = (int)N;
         while (mc > 1 && mfma_lds_bytes((int)K, mc, 16) > max_lds) mc = (mc + 1) / 2;
         if (mfma_lds_bytes((int)K, mc, 16) <= max_lds && (okern == 4 || mc == N))
-            return pick_geometry_mfma(di, K, M, mc, owgs);
+            return pick_geometry_mfma(di, K, M, mc, owgs, owaves);
     }
     g.grid = owgs > 0 ? owgs : grid_per_matrix(cus, mats, M);
     // One column with rows of at most 8192 values and ~500 KB or more of
@@ -1239,7 +1247,7 @@ static int launch_gemv(DeviceInfo *di, const Geometry &geo, GemvParams p, int nc
         if (geo.mfma_ga && (p.x || !p.y)) return Q4K_EINVAL;  // GA reads the Q8_1 buffer
         fn = geo.mfma_ga ? (p.sums ? q4k_mfma_ga_sums_kernel(nc, geo.waves, geo.slots)
                                    : q4k_mfma_ga_kernel(nc, geo.waves, geo.slots))
-                         : q4k_mfma_kernel(nc, p.sums != nullptr);
+                         : q4k_mfma_kernel(nc, geo.waves, p.sums != nullptr);
         p.rows_base = geo.rows_base;
         p.rows_extra = geo.rows_extra;
         p.rpw = geo.ks;

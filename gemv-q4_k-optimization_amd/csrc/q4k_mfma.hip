@@ -7,23 +7,24 @@
 
 namespace q4k {
 
-template <bool SUMS>
+template <int WAVES, bool SUMS>
 static const void *mfma_kernel_nc(int nc) {
     switch (nc) {
-        case 1: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<1, 8, SUMS>);
-        case 2: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<2, 8, SUMS>);
-        case 3: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<3, 8, SUMS>);
-        case 4: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<4, 8, SUMS>);
-        case 5: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<5, 8, SUMS>);
-        case 6: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<6, 8, SUMS>);
-        case 7: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<7, 8, SUMS>);
-        case 8: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<8, 8, SUMS>);
+        case 1: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<1, WAVES, SUMS>);
+        case 2: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<2, WAVES, SUMS>);
+        case 3: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<3, WAVES, SUMS>);
+        case 4: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<4, WAVES, SUMS>);
+        case 5: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<5, WAVES, SUMS>);
+        case 6: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<6, WAVES, SUMS>);
+        case 7: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<7, WAVES, SUMS>);
+        case 8: return reinterpret_cast<const void *>(&gemv_q4k_mfma_kernel<8, WAVES, SUMS>);
         default: return nullptr;
     }
 }
 
-const void *q4k_mfma_kernel(int nc, bool sums) {
-    return sums ? mfma_kernel_nc<true>(nc) : mfma_kernel_nc<false>(nc);
+const void *q4k_mfma_kernel(int nc, int waves, bool sums) {
+    if (waves > 8) return sums ? mfma_kernel_nc<16, true>(nc) : mfma_kernel_nc<16, false>(nc);
+    return sums ? mfma_kernel_nc<8, true>(nc) : mfma_kernel_nc<8, false>(nc);
 }
 
 template <int NIF>

@@ -92,7 +92,7 @@ const void *q6k_sums_kernel(int nc, int waves, int pro, int slots, bool dense);
 // The matrix-core kernels (q4k_mfma.hip, q6k_mfma.hip) for nc columns
 // (sums: the parity variant); ga: the A operand from the Q8_1 buffer, nif
 // items in flight per wave.
-const void *q4k_mfma_kernel(int nc, bool sums);
+const void *q4k_mfma_kernel(int nc, int waves, bool sums);
 const void *q4k_mfma_ga_kernel(int nc, int waves, int nif);
 const void *q6k_mfma_kernel(int nc, int waves);
 const void *q6k_mfma_ga_kernel(int nc, int waves);

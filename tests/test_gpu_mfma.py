@@ -88,7 +88,8 @@ def test_mfma_kernel_zero_inputs(Q, O, gpu):
 def test_mfma_result_independent_of_work_split(Q, O, gpu, M, K, N):
     """The summation order depends on K alone: launches over 256, 64, 16 and
     4 workgroups (8, 4, 2 and 1 waves per tile, one to several rounds), the
-    8-wave variant and row slices at odd offsets give the same bits."""
+    16-wave variant (waves_per_wg 9 to 16; 8 waves are automatic) and row
+    slices at odd offsets give the same bits."""
     import torch
     wq, x = inputs(Q, M, K, N, seed=23)
     wd, xd = to_dev(wq, gpu), to_dev(x, gpu)
@@ -96,16 +97,17 @@ def test_mfma_result_independent_of_work_split(Q, O, gpu, M, K, N):
     try:
         Q.set_geometry_override(kernel=4)
         y = Q.mul_mat_vec_q(wd, K, xd)
-        _, sums16, _ = Q.mul_mat_vec_q_sums(wd, K, xd)
+        _, sums8, _ = Q.mul_mat_vec_q_sums(wd, K, xd)
+        assert Q.geometry(K, M, N)["waves_per_wg"] == 8
         for wgs in (64, 16, 4):
             Q.set_geometry_override(kernel=4, workgroups=wgs)
             assert torch.equal(Q.mul_mat_vec_q(wd, K, xd), y), f"{wgs} workgroups"
-        for wgs in (0, 16):
-            Q.set_geometry_override(kernel=4, waves_per_wg=8, workgroups=wgs)
-            assert Q.geometry(K, M, N)["waves_per_wg"] == 8
-            assert torch.equal(Q.mul_mat_vec_q(wd, K, xd), y), f"8 waves, {wgs} workgroups"
+        for waves, wgs in ((16, 0), (16, 16), (9, 7), (8, 16)):
+            Q.set_geometry_override(kernel=4, waves_per_wg=waves, workgroups=wgs)
+            assert Q.geometry(K, M, N)["waves_per_wg"] == (16 if waves > 8 else 8)
+            assert torch.equal(Q.mul_mat_vec_q(wd, K, xd), y), f"{waves} waves, {wgs} workgroups"
             ys, sums, _ = Q.mul_mat_vec_q_sums(wd, K, xd)
-            assert torch.equal(ys, y) and torch.equal(sums, sums16)
+            assert torch.equal(ys, y) and torch.equal(sums, sums8)
         Q.set_geometry_override(kernel=4)
         cut = M // 3 + 5
         top = Q.op_mul_mat_vec_q(wd[:cut], K, q8d, N, row_low=0, row_high=cut)
