@@ -78,22 +78,42 @@ def test_division_by_127_identity(O):
     assert ((a * rcp).astype(np.float32) != a / np.float32(127)).sum() > 1000
 
 
-def _fast_round_agrees(d, xs, threshold):
-    """The in-launch quantiser's fast rounding: y = x * r with r any float
-    within one ulp of 1/d (the accuracy of v_rcp_f32), rint(y) accepted when
-    |y - rint(y)| <= threshold.  Returns the number of accepted values whose
-    rint(y) differs from ggml's roundf(x / d) (IEEE quotient)."""
+def _rounded_sum(x, r):
+    """fma(x, r, 1.5 * 2^23) in float32: x * r (at most 48 bits) plus the
+    constant is formed in float64, where only bits below 2^-29 of the sum can
+    be lost; a sum that lands on a half-integer that way is moved back to its
+    side of it, so that the second rounding is that of the exact sum."""
+    magic = 12582912.0
+    p = x.astype(np.float64) * r.astype(np.float64)  # exact: 24 + 24 bits
+    s = p + magic
+    lost = p - (s - magic)  # exact
+    tie = s - np.floor(s) == 0.5
+    s = np.where(tie & (lost > 0), np.nextafter(s, np.inf), s)
+    s = np.where(tie & (lost < 0), np.nextafter(s, -np.inf), s)
+    return s.astype(np.float32)
+
+
+def _bounded_round_wrong(d, xs, below, above):
+    """The in-launch quantiser's rounding: r any float within one ulp of 1/d
+    (the accuracy of v_rcp_f32), the bounds r0 = r (1 - below) and r1 = r
+    (1 + above) rounded to float32, one fma with each onto 1.5 * 2^23; where
+    both sums agree their low byte is the q8.  Returns (the number of agreeing
+    values whose byte differs from ggml's roundf(x / d) with the IEEE
+    quotient, the share of values that do not agree)."""
     d = np.float32(d)
-    r0 = np.float32(1.0) / d
-    bad = 0
-    q_ref = np.float32(xs / d)
-    q_ref = np.sign(q_ref) * np.floor(np.abs(q_ref) + np.float32(0.5))
-    for r in (r0, np.nextafter(r0, np.float32(0)), np.nextafter(r0, np.float32(np.inf))):
-        y = (xs * r).astype(np.float32)
-        ry = np.rint(y)
-        fast = np.abs(y - ry) <= threshold
-        bad += int(np.sum(fast & (ry != q_ref)))
-    return bad
+    q = np.float32(xs / d)
+    q_ref = (np.sign(q) * np.floor(np.abs(q) + np.float32(0.5))).astype(np.int64) & 0xFF
+    near = np.float32(1.0) / d
+    wrong, differ = 0, 0
+    for r in (near, np.nextafter(near, np.float32(0)), np.nextafter(near, np.float32(np.inf))):
+        if abs(float(r) * float(d) - 1.0) > 2.0 ** -23:
+            continue  # further than one ulp from 1/d
+        m0 = _rounded_sum(xs, np.float32(r * np.float32(1.0 - below))).view(np.uint32)
+        m1 = _rounded_sum(xs, np.float32(r * np.float32(1.0 + above))).view(np.uint32)
+        same = m0 == m1
+        wrong += int(np.sum(same & ((m0 & 0xFF) != q_ref)))
+        differ += int(np.sum(~same))
+    return wrong, differ / (3 * xs.size)
 
 
 def _tie_adversaries(rng, d, n=4000):
@@ -103,22 +123,41 @@ def _tie_adversaries(rng, d, n=4000):
     return (np.float32(d) * (k + off)).astype(np.float32)
 
 
-def test_fast_rounding_threshold_is_safe():
-    """|y - x/d| <= 127 (2^-23 + 2^-24) < 2^-15.4 and |fl(x/d) - x/d| <= 2^-17,
-    so rint(y) = roundf(fl(x/d)) whenever y is more than 2^-15 from a
-    half-integer; the kernel accepts up to 0.5 - 2^-14 (twice that margin).
-    Checked over random and near-tie quotients with the three reciprocals a
-    one-ulp rcp can return; a threshold without the margin fails."""
+def test_bounded_rounding_is_safe():
+    """quantize_lanes takes a byte only where the sums with both bounds agree:
+    r is within 2^-23 of 1/d, the bounds' own rounding and the quotient's are
+    2^-24 each, so bounds 1.25 and 1.5 * 2^-22 from r hold the rounded quotient
+    strictly between them.  Over random and near-tie quotients, block maxima
+    from 2^-100 (below which the kernel divides) to 2^57 and the reciprocals a
+    one-ulp rcp can return no agreeing byte is wrong; bounds that allow for
+    none of those errors are wrong somewhere; and on ordinary values few
+    disagree (the kernel's exact path)."""
     rng = np.random.default_rng(42)
-    thr = np.float32(0.5 - 2.0 ** -14)
-    too_loose = np.float32(0.5 - 2.0 ** -19)
-    loose_bad = 0
-    for _ in range(300):
-        amax = np.float32(np.exp(rng.uniform(-40, 40)))
+    tight_wrong = 0
+    for i in range(300):
+        amax = np.float32(2.0 ** rng.uniform(-100, 57))
         d = np.float32(amax / np.float32(127.0))
-        xs = np.concatenate([rng.uniform(-1, 1, 2000).astype(np.float32) * amax,
-                             _tie_adversaries(rng, d)]).astype(np.float32)
+        plain = rng.uniform(-1, 1, 2000).astype(np.float32) * amax
+        xs = np.concatenate([plain, _tie_adversaries(rng, d)]).astype(np.float32)
         xs = xs[np.abs(xs) <= amax]
-        assert _fast_round_agrees(d, xs, thr) == 0
-        loose_bad += _fast_round_agrees(d, xs, too_loose)
-    assert loose_bad > 0
+        assert _bounded_round_wrong(d, xs, 1.25 * 2.0 ** -22, 1.5 * 2.0 ** -22)[0] == 0
+        assert _bounded_round_wrong(d, plain, 1.25 * 2.0 ** -22, 1.5 * 2.0 ** -22)[1] < 0.01
+        tight_wrong += _bounded_round_wrong(d, xs, 0.0, 2.0 ** -23)[0]
+    assert tight_wrong > 0
+
+
+def test_bounded_rounding_on_generic_ties():
+    """The values next to every tie of blocks whose d is no power of two: x
+    from a few floats below (k + 1/2) d to a few above, so that the IEEE
+    quotient falls on, just under and just over the half-integer."""
+    rng = np.random.default_rng(43)
+    for _ in range(40):
+        d = np.float32(np.float32(2.0 ** rng.uniform(-20, 20)) / np.float32(127.0))
+        ties = ((np.arange(-127, 127) + 0.5) * np.float64(d)).astype(np.float32)
+        steps = [ties]
+        up, down = ties, ties
+        for _ in range(6):
+            up, down = np.nextafter(up, np.float32(np.inf)), np.nextafter(down, np.float32(-np.inf))
+            steps += [up, down]
+        xs = np.concatenate(steps)
+        assert _bounded_round_wrong(d, xs, 1.25 * 2.0 ** -22, 1.5 * 2.0 ** -22)[0] == 0
