@@ -434,10 +434,11 @@ __device__ __forceinline__ float lane_amax(const float (&v)[V]) {
 // One fma for each bound adds 1.5 * 2^23, which rounds to the integer (ties to
 // even) and leaves it in the low mantissa bits: where the two agree no
 // half-integer lies between the bounds (one may be the lower or the upper
-// bound itself; the quotient lies strictly inside) and the low byte is the
-// answer (a q8 in [-127, 127] is the sum's low byte).  So a value takes two fmas, one bit operation that collects the
-// differences (a chain per dword) and 3/4 of a byte permute.  A block of zeros
-// passes: 0 * inf is the default NaN, low byte 0.  Where a lane of the wave has
+// bound itself; the quotient of a v other than 0 lies strictly inside) and the
+// low byte is the answer (a q8 in [-127, 127] is the sum's low byte; v = 0
+// gives 0 at both bounds).  So a value takes two fmas, one bit operation that
+// collects the differences (a chain per dword) and 3/4 of a byte permute.  A
+// block of zeros passes: 0 * inf is the default NaN, low byte 0.  Where a lane of the wave has
 // a value whose bounds differ (one value in ~4 * 10^4), a NaN, or an amax so
 // small that r could overflow, the wave starts again with the exact division
 // (an infinite amax: d is a NaN and every byte 0 either way).  Bounds 8 * 2^-22
@@ -451,6 +452,11 @@ __device__ __forceinline__ void quantize_lanes(const float (&v)[V], float &d, ui
     const float lane_max = lane_amax<true>(v);
     const float amax = block_max<LPB>(lane_max);  // (without the lanes that hold a NaN)
     d = div127(amax);
+    // (collected here, where it leaves no register across the rounding: one more
+    // than 64 took the tile kernel's second workgroup per CU, and a pre-quantised
+    // 20012 x 8448 from 22.4 to 25.2 us)
+    const bool tiny = __builtin_bit_cast(uint32_t, amax) - 1u < __builtin_bit_cast(uint32_t, 0x1p-100f) - 1u;  // but not 0
+    const uint64_t odd = __builtin_amdgcn_ballot_w64(lane_max != lane_max || tiny);
     const float r = __builtin_amdgcn_rcpf(d);
     const float r0 = r * (1.0f - 0x1.4p-22f), r1 = r * (1.0f + 0x1.8p-22f);
     uint32_t differ[V / 4];
@@ -473,9 +479,7 @@ __device__ __forceinline__ void quantize_lanes(const float (&v)[V], float &d, ui
     uint32_t any = differ[0];
 #pragma unroll
     for (int w = 1; w < V / 4; ++w) any |= differ[w];
-    // 0 < amax < 2^-100
-    const bool tiny = __builtin_bit_cast(uint32_t, amax) - 1u < __builtin_bit_cast(uint32_t, 0x1p-100f) - 1u;
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(any != 0 || lane_max != lane_max || tiny) != 0, 0)) {
+    if (__builtin_expect((__builtin_amdgcn_ballot_w64(any != 0) | odd) != 0, 0)) {
         const float exact_max = block_max<LPB>(lane_amax<false>(v));
         d = div127(exact_max);
         const float dd = exact_max == 0.0f ? 1.0f : d;  // (then the values are zeros and NaNs)
