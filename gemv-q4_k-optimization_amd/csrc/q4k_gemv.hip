@@ -946,12 +946,12 @@ static Geometry pick_geometry(const DeviceInfo &di, int64_t K, int64_t M, int64_
     // pre-quantised route, up to 8 columns in one launch
     if (q81 && !fused && mats == 1 && N <= kMfmaCols &&
         (okern == 6 || (okern == 0 && use_mfma_ga(M, N, K) &&
-                         !(use_mfma(M, N, K) && mfma_lds_bytes((int)K, (int)N, 16) <= max_lds))))
+                         !(use_mfma(M, N, K) && mfma_lds_bytes((int)K, (int)N, mfma_waves(owaves)) <= max_lds))))
         return pick_geometry_mfma(di, K, M, (int)N, owgs, owaves, true);
     if (!fused && mats == 1 && (okern == 4 || (okern == 0 && use_mfma(M, N, K)))) {
         int mc = (int)N;
-        while (mc > 1 && mfma_lds_bytes((int)K, mc, 16) > max_lds) mc = (mc + 1) / 2;
-        if (mfma_lds_bytes((int)K, mc, 16) <= max_lds && (okern == 4 || mc == N))
+        while (mc > 1 && mfma_lds_bytes((int)K, mc, mfma_waves(owaves)) > max_lds) mc = (mc + 1) / 2;
+        if (mfma_lds_bytes((int)K, mc, mfma_waves(owaves)) <= max_lds && (okern == 4 || mc == N))
             return pick_geometry_mfma(di, K, M, mc, owgs, owaves);
     }
     g.grid = owgs > 0 ? owgs : grid_per_matrix(cus, mats, M);

@@ -35,7 +35,8 @@
 // lane gets the min sums of its own four sub-blocks, as it gets their S.
 //
 // Work split: tiles of 16 rows, split evenly over the workgroups (one per
-// CU, 8 or 16 waves).  The waves of a workgroup form 8/KS groups of KS waves; in
+// CU, 8 or, by override, 16 waves).  The waves of a workgroup form groups of KS
+// (8/KS groups of 8 waves); in
 // each round every group takes one tile and its KS waves take equal shares
 // of the tile's super-blocks.  At the end of a round each wave leaves its
 // partial results in LDS and, after a barrier, the workgroup combines the KS
@@ -49,8 +50,8 @@
 // of column c / 18), goes to a second LDS slot of the wave as it lies in
 // memory, and the MFMA lanes read their A operands from there.  The LDS
 // holds only the d8 of every (block, column) besides, so the length of the
-// rows is not bounded by the LDS (eight 14336-value columns staged would
-// take 166 KB of its 160).  The sums of the blocks' q8, which the staged
+// rows is not bounded by the LDS (staged, eight columns end at 14336 values,
+// 163456 of its 163840 bytes).  The sums of the blocks' q8, which the staged
 // layout keeps times d8, come from MFMAs of the same registers as the B
 // operand against an A of ones (D[i][j] = the sum of column j % 8's block
 // 4h + p + 2(j/8), in every row i); d8 * that sum is the staged product, so

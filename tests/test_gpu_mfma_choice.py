@@ -40,3 +40,8 @@ def test_choice_against_oracle_and_between_routes(Q, O, gpu, wtype, M, K, N):
     ws = torch.empty(Q.q8_1_bytes(K, N), dtype=torch.uint8, device=gpu)
     assert torch.equal(Q.mul_mat_vec_q(wd, K, xd, workspace=ws, wtype=wtype), y)
     assert torch.equal(Q.op_mul_mat_vec_q(wd, K, Q.quantize_row_q8_1(xd), N, wtype=wtype), y)
+
+
+def test_staged_kernel_up_to_the_end_of_the_lds(Q, gpu):
+    """Eight columns of 14336 values fit beside eight waves (163456 of 163840 bytes)."""
+    assert Q.geometry(14336, 8192, 8)["kernel"] == 4
