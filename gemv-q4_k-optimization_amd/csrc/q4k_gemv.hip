@@ -235,63 +235,102 @@ static int tile_lds_bytes(int K, int nc, int waves) {
 }
 static int lds_bytes_linear(int K) { return K + K / 4; }
 
+// The share in percent of the matrix-core kernel's tile slots that hold a tile
+// (8 waves): a workgroup's tiles go in rounds of a power of two of them, so five
+// take the time of eight.
+int mfma_fill(int64_t tiles, int cus) {
+    const int64_t nt = (tiles + cus - 1) / cus;
+    int64_t groups = 1;
+    while (groups < 8 && 2 * groups <= nt) groups *= 2;
+    return (int)(100 * tiles / (cus * ((nt + groups - 1) / groups * groups)));
+}
+
+// Rows per CU up to which five columns or more of rows longer than 5120 values
+// stay with the column split; beyond, the matrix-core kernels (five columns up to
+// 8192 values: the tile kernel, until use_mfma takes them).  us per op, MI355X,
+// column split against what follows: N=5 (tile) 2560 x 8192 10.3 against 11.1, 2304
+// x 5376 8.1 / 8.4, 2816 x 6144 10.0 / 9.5; N=6 2816 x 6144 10.8 / 9.7, 2816 x 8192
+// 11.9 / 12.5; N=8 2304 x 6144 10.6 / 11.3, 2816 x 8192 13.5 / 13.3; longer, on the
+// Q8_1 copy: N=5 2304 x 9472 11.0 / 13.2, 2816 x 12800 17.0 / 15.7, N=7 2064 x 9472
+// 14.4 / 13.5, N=5 2064 x 22272 21.2 / 21.0.
+static int64_t split_rows_per_cu(int64_t N, int64_t K) {
+    if (K > 8192) return N >= 7 || K > 16384 ? 8 : 10;
+    if (N == 5) return K == 8192 ? 12 : 10;
+    return N == 6 && K > 6144 ? 12 : 10;
+}
+
 // Where the automatic choice is the matrix-core kernel (us per op, MI355X,
 // matrix-core against the choice without it).  It costs the same from one to
 // eight columns, so it pays where the tile kernel's work per column, or the
 // lanes it leaves idle on rows shorter than 16 super-blocks, have grown past
-// that.
+// that -- and, near the line, only where its rounds are full (mfma_fill: 18944
+// rows are 4.6 tiles per CU in 8 slots, 58 %).
 //  - rows of one or two super-blocks (up to 512 values), which have no short
-//    teams: two columns and more from 256 row tiles: 65536 x 512 N=3 9.34
-//    against 22.1, 8192 x 512 N=2 4.55 / 5.45, 65536 x 256 N=2 7.15 / 17.5
-//    (2048 x 512 N=4 4.37 / 4.04: not with fewer).
-//  - rows of 3 to 13: five columns and more from 256 tiles: 65536 x 1024 N=8
-//    13.4 / 39.2, 32768 x 768 N=5 8.18 / 17.4, 4096 x 2048 N=6 5.43 / 6.44,
-//    24576 x 3328 N=5 16.9 / 17.2 (2048 x 768 N=6 5.42 / 4.41, 2048 x 2560 N=6
-//    6.14 / 5.77).  Three and four columns only from 9 super-blocks on (rows
-//    of 3 to 8 run in short teams there): four from 1024 tiles, three from
-//    2048: 16384 x 2304 N=4 9.39 / 10.5, 32768 x 2304 N=3 13.3 / 15.4 (8192 x
-//    3328 N=4 8.29 / 8.10, 16384 x 2560 N=3 9.39 / 9.27).
-//  - rows of 14 to 16: eight columns from 896 tiles and six to eight from 4096
-//    (14336 x 4096 N=8 13.1 / 16.6, 128256 x 4096 N=8 64.6 / 87.3); with fewer
-//    rows or columns the tile kernel is within a few percent either way
-//    (4096 x 4096 N=8 8.4 / 8.8, N=5 7.3 / 7.2; 14336 x 4096 N=4 11.8 / 10.9).
-//  - rows of up to 5120 values: six columns from 512 tiles, five from 864
-//    (13824 x 5120 N=6 15.0 / 20.9); of up to 8192 (where the tile kernel
-//    reads every column's activation from LDS at each step): six from just
-//    over 8 rows per CU, five from 512 tiles: 4096 x 8192 N=8 13.8 / 15.8, N=6
-//    13.0 / 13.7, 8192 x 6144 N=5 12.0 / 14.0 (3072 x 8192 N=5 11.4 / 11.2);
-//    longer ones as those of 5120: with fewer rows the kernel below is the
-//    better one (4096 x 11008 N=6 15.6 against 15.0).
+//    teams: three columns and more from 256 row tiles, two from 288: 65536 x 512
+//    N=3 9.34 against 22.1, 8192 x 512 N=2 4.55 / 5.45, 65536 x 256 N=2 7.15 /
+//    17.5 (2048 x 512 N=4 4.37 / 4.04: not with fewer).
+//  - rows of 3 to 8: five columns and more from 256 tiles: 65536 x 1024 N=8 13.4 /
+//    39.2, 32768 x 768 N=5 8.18 / 17.4, 4096 x 2048 N=6 5.43 / 6.44 (2048 x 768
+//    N=6 5.42 / 4.41).
+//  - rows of 9 to 13, where the rounds are full enough (the fewer columns, the
+//    fuller): 16384 x 2304 N=4 9.33 / 10.2, 26624 x 3072 N=4 15.3 / 16.1, 24576 x
+//    2816 N=5 15.2 / 15.4, 32768 x 2304 N=3 13.0 / 14.4; not 18944 x 3072 N=4 14.6
+//    / 12.3, N=5 14.8 / 13.7, 8960 x 3328 N=5 10.6 / 9.4, 47367 x 2816 N=3 21.7 /
+//    18.6, 16526 x 3072 N=7 (half full) 15.9 / 15.2.
+//  - rows of 16: eight columns from 896 tiles and six to eight from 4096 (14336 x
+//    4096 N=8 13.1 / 16.6, 128256 x 4096 N=8 64.6 / 87.3); with fewer rows or
+//    columns the tile kernel is within a few percent either way (4096 x 4096 N=8
+//    8.4 / 8.8, N=5 7.3 / 7.2; 14336 x 4096 N=4 11.8 / 10.9).  Rows of 14 and 15:
+//    the tile kernel (18944 x 3584 N=8 17.7 with it, 18.7 with an earlier form of
+//    this kernel, for which the lines from 3584 to 5120 values were drawn;
+//    test_automatic_choice holds them).
+//  - rows of up to 5120 values: six columns from 512 tiles, five from 864 (13824 x
+//    5120 N=6 15.0 / 20.9); of up to 8192 (where the tile kernel reads every
+//    column's activation from LDS at each step): six and more past the column
+//    split (split_rows_per_cu), five from 512 tiles: 4096 x 8192 N=8 13.8 / 15.8,
+//    8192 x 6144 N=5 12.0 / 14.0, below 512 tiles of the longer ones only where the
+//    rounds are full (5120 x 8192 N=6 15.2 / 14.0, 4608 x 7168 N=6 14.0 / 13.8);
+//    longer ones as those of 5120: with fewer rows the kernel below.
 // Rows whose columns do not fit the LDS in one launch are left to the others.
-static bool use_mfma(int64_t M, int64_t N, int64_t K) {
+static bool use_mfma(int64_t M, int64_t N, int64_t K, int cus) {
     const int64_t tiles = (M + kMfmaRows - 1) / kMfmaRows;
-    if (K <= 512) return N >= 2 && tiles >= 256;
+    const int fill = mfma_fill(tiles, cus);
+    if (K <= 512) return N >= 2 && tiles >= (N == 2 ? 288 : 256);
+    if (K < 2304) return N >= 5 && tiles >= 256;
     if (K < 3584) {
-        if (N >= 5) return tiles >= 256;
-        return K >= 2304 && ((N == 4 && tiles >= 1024) || (N == 3 && tiles >= 2048));
+        const bool last = K == 3328;
+        if (N == 3) return tiles >= 1900 && fill >= (K <= 2560 ? 87 : 93) && K <= 2816;
+        if (N == 4) return tiles >= 1024 && fill >= (last ? 93 : 80);
+        if (N == 5) return tiles >= 256 && fill >= (last ? 80 : 75);
+        if (N == 6) return tiles >= 256 && fill >= (last ? 75 : 65);
+        if (N == 7) return tiles >= 256 && fill >= 55;
+        return N == 8 && tiles >= 256;
     }
     if (K <= 4096) return K == 4096 && ((N == 8 && tiles >= 896) || (N >= 6 && tiles >= 4096));
     if (K <= 5120) return (N >= 6 && tiles >= 512) || (N == 5 && tiles >= 864);
-    if (K <= 8192) return (N >= 6 && tiles > 128) || (N == 5 && tiles >= 512);
+    if (K <= 8192) {
+        if (N == 5) return tiles >= 864 || (tiles >= 512 && fill >= 60);
+        if (N < 6 || M <= split_rows_per_cu(N, K) * cus) return false;
+        const int full = K <= 6144 ? 0 : N == 6 ? (K <= 7168 ? 65 : 87) : (N == 7 && K > 7168 ? 65 : 0);
+        return tiles >= 512 || fill >= full;
+    }
     return (N >= 6 && tiles >= 512) || (N == 5 && tiles >= 864);
 }
 
 // Where the pre-quantised route runs the matrix-core kernel with its A
 // operand read from the Q8_1 buffer (GA): rows longer than 8192 values, five to
-// eight columns, more than 8 rows per CU (below, the column split), where (the
-// caller checks) the staged matrix-core kernel is not chosen or cannot hold
-// the columns.  Measured on MI355X (us per op with a Q8_1 workspace, the
-// quantiser launch included; GA against the tile kernel): 4096 x 14336 N=8
-// 18.7 against 23, 8192 x 28672 N=8 44 / 67; against the column split, 3072 x
-// 14336 N=7 17.2 / 23.5, 2432 x 9472 N=7 13.7 / 15.8, 3072 x 22272 N=7 22.9 /
-// 35.3, 3072 x 28672 N=5 25.2 / 30.8 (2048 x 14336 N=6 16.3 / 16.1, 1024 x
-// 22272 N=7 21.5 / 16.6: not with fewer rows).  Slower at four columns (8192 x
-// 28672 39.4 / 37.6).  Two items in flight per wave, not four (4096 x 14336
-// N=8 15.1 against 17.0, quantised before); weights through the slot, not
-// loaded straight into the lanes' registers in MFMA order (N=6 17.6 / 21.4).
-static bool use_mfma_ga(int64_t M, int64_t N, int64_t K) {
-    const int64_t tiles = (M + kMfmaRows - 1) / kMfmaRows;
-    return K > 8192 && N >= 5 && tiles > 128;
+// eight columns, past the column split (split_rows_per_cu), where (the caller
+// checks) the staged matrix-core kernel is not chosen or cannot hold the columns.
+// Measured on MI355X (us per op with a Q8_1 workspace, the quantiser launch
+// included; GA against the tile kernel): 4096 x 14336 N=8 18.7 against 23, 8192 x
+// 28672 N=8 44 / 67; against the column split, 3072 x 14336 N=7 17.2 / 23.5, 3072
+// x 22272 N=7 22.9 / 35.3, 3072 x 28672 N=5 25.2 / 30.8 (1024 x 22272 N=7 21.5 /
+// 16.6: not with fewer rows).  Slower at four columns (8192 x 28672 39.4 / 37.6).
+// Two items in flight per wave, not four (4096 x 14336 N=8 15.1 against 17.0,
+// quantised before); weights through the slot, not loaded straight into the
+// lanes' registers in MFMA order (N=6 17.6 / 21.4).
+static bool use_mfma_ga(int64_t M, int64_t N, int64_t K, int cus) {
+    return K > 8192 && N >= 5 && M > split_rows_per_cu(N, K) * cus;
 }
 
 // Waves per workgroup of the matrix-core kernel: 8 (16 measured slower from few
@@ -794,7 +833,7 @@ static bool ksplit_nc_auto(int64_t K, int64_t M, int64_t N, int cus, int &tr, in
 // 6.64.  Not at 4096 rows (4096 x 4096 N=2 4.86 -> 5.08, N=4 6.29 -> 6.42)
 // nor beyond; two columns only up to 8 rows per CU (2048 x 4096: 4.12 ->
 // 4.11).
-bool split_columns(int64_t K, int64_t M, int64_t N, int cus) {
+bool split_columns(int64_t K, int64_t M, int64_t N, int cus, bool q6) {
     if (N < 2 || N > Q4K_MAX_BATCH || cus < 1) return false;
     const int64_t rho = (M + cus - 1) / cus;
     // rows shorter than one group of 5 or more blocks: up to 4 rows per CU
@@ -803,10 +842,11 @@ bool split_columns(int64_t K, int64_t M, int64_t N, int cus) {
     // 5.79 / 4.44, N=2 4.35 / 4.06, 2048 x 2304 N=2 4.08 / 3.86, Q6_K 2048 x
     // 2048 N=3 4.81 / 4.26; at up to 4 the split: 512 x 2048 N=4 3.08 / 4.04,
     // 1024 x 2560 N=4 4.18 / 4.53)
-    const int64_t lim = K < 4096 && K > 1024 ? 4 : (N == 2 ? 8 : 12);
-    // five columns or more of long rows: up to 8 rows per CU (beyond, the
-    // matrix-core kernels: use_mfma, use_mfma_ga, use_mfma_q6)
-    if (N >= 5 && K > 5120 && rho > 8) return false;
+    // five columns or more of long rows: up to where the matrix-core kernels
+    // take over (Q6_K: 8 rows per CU, 3072 x 14336 N=7 39.6 against 18.7)
+    const int64_t lim = K < 4096 && K > 1024 ? 4
+                        : N >= 5 && K > 5120 ? (q6 ? 8 : split_rows_per_cu(N, K))
+                                             : (N == 2 ? 8 : 12);
     return rho <= lim && K <= 8 * 4096 && (K >= 4096 || ksplit_short_rows(K));
 }
 
@@ -848,7 +888,7 @@ static Geometry pick_geometry(const DeviceInfo &di, int64_t K, int64_t M, int64_
     // several columns over few rows: one-column channels (automatic only;
     // where the aligned F32 column takes the K-split kernel, so both routes
     // decide alike)
-    if (!fused && mats == 1 && okern == 0 && orows == 0 && owaves == 0 && owgs == 0 && split_columns(K, M, N, cus) &&
+    if (!fused && mats == 1 && okern == 0 && orows == 0 && owaves == 0 && owgs == 0 && split_columns(K, M, N, cus, false) &&
         pick_geometry(di, K, M, 1, 0, N, true, false).ksplit) {
         Geometry g1 = pick_geometry(di, K, M, 1, 0, N, f32_vec, q81);
         g1.colsplit = (int)N;
@@ -944,15 +984,14 @@ static Geometry pick_geometry(const DeviceInfo &di, int64_t K, int64_t M, int64_
     }
     // the matrix-core kernel with its A operand from the Q8_1 buffer: the
     // pre-quantised route, up to 8 columns in one launch
+    auto mfma_fits = [&](int n) { return mfma_lds_bytes((int)K, n, mfma_waves(owaves)) <= max_lds; };
     if (q81 && !fused && mats == 1 && N <= kMfmaCols &&
-        (okern == 6 || (okern == 0 && use_mfma_ga(M, N, K) &&
-                         !(use_mfma(M, N, K) && mfma_lds_bytes((int)K, (int)N, mfma_waves(owaves)) <= max_lds))))
+        (okern == 6 || (okern == 0 && use_mfma_ga(M, N, K, cus) && !(use_mfma(M, N, K, cus) && mfma_fits((int)N)))))
         return pick_geometry_mfma(di, K, M, (int)N, owgs, owaves, true);
-    if (!fused && mats == 1 && (okern == 4 || (okern == 0 && use_mfma(M, N, K)))) {
+    if (!fused && mats == 1 && (okern == 4 || (okern == 0 && use_mfma(M, N, K, cus)))) {
         int mc = (int)N;
-        while (mc > 1 && mfma_lds_bytes((int)K, mc, mfma_waves(owaves)) > max_lds) mc = (mc + 1) / 2;
-        if (mfma_lds_bytes((int)K, mc, mfma_waves(owaves)) <= max_lds && (okern == 4 || mc == N))
-            return pick_geometry_mfma(di, K, M, mc, owgs, owaves);
+        while (mc > 1 && !mfma_fits(mc)) mc = (mc + 1) / 2;
+        if (mfma_fits(mc) && (okern == 4 || mc == N)) return pick_geometry_mfma(di, K, M, mc, owgs, owaves);
     }
     g.grid = owgs > 0 ? owgs : grid_per_matrix(cus, mats, M);
     // One column with rows of at most 8192 values and ~500 KB or more of

@@ -121,7 +121,9 @@ int run_gemv_q6(const void *src0, int64_t ne00, int64_t ne01, int64_t nb01, cons
 
 // Whether N columns of an (M, K) product run as one launch of N one-column
 // channels (q4k_gemv.hip: the measured rule), on cus CUs.
-bool split_columns(int64_t K, int64_t M, int64_t N, int cus);
+bool split_columns(int64_t K, int64_t M, int64_t N, int cus, bool q6);
+// How full the matrix-core kernels' rounds are, in percent (q4k_gemv.hip)
+int mfma_fill(int64_t tiles, int cus);
 
 // Workgroups per weight matrix of a launch over `mats` matrices of M rows:
 // the CUs shared among the matrices, at least one, at most one per row; 16

@@ -309,31 +309,52 @@ static bool q6_ksplit_auto(int64_t K, int64_t M, int cus, int &tr, int &waves, i
 
 // Where the matrix-core kernel is chosen (all columns in one launch, which
 // the caller checks); us per op on MI355X, matrix-core against the choice
-// without it, as for Q4_K (use_mfma).
+// without it, as for Q4_K (use_mfma), near the lines where its rounds are full
+// (mfma_fill).
 //  - rows of one or two super-blocks: three columns and more from 256 row tiles:
 //    65536 x 512 N=3 11.7 against 33.2, 8192 x 512 N=8 5.16 / 10.1.
-//  - rows of 3 to 12: five columns and more from 256 tiles, four from 9
-//    super-blocks and 1024 tiles: 32768 x 768 N=5 10.2 / 23.8, 4096 x 1536 N=6
-//    6.60 / 7.30, 4096 x 2048 N=8 6.66 / 8.57, 16384 x 2560 N=4 11.8 / 13.6, 6144
-//    x 2560 N=8 9.39 / 10.4, 4096 x 3072 N=6 7.87 / 8.44 (2048 x 768 N=6 5.94 /
-//    4.32).  Of 13: six and more (24576 x 3328 N=5 23.0 / 20.8).
+//  - rows of 3 to 8: five columns and more from 256 tiles: 32768 x 768 N=5 10.2 /
+//    23.8, 4096 x 1536 N=6 6.60 / 7.30, 4096 x 2048 N=8 6.66 / 8.57 (2048 x 768 N=6
+//    5.94 / 4.32).
+//  - rows of 9 to 12: the fewer columns, the fuller: 16384 x 2560 N=4 11.8 / 13.6,
+//    26624 x 2816 N=5 20.8 / 21.8, 12288 x 3072 N=6 13.4 / 14.0; not 18944 x 3072
+//    N=5 20.8 / 17.2, 6144 x 2816 N=5 9.14 / 8.67, 8768 x 3072 N=5 14.7 / 12.7.  Of
+//    13: six and more (24576 x 3328 N=5 23.0 / 20.8; 18944 x 3328 N=6 22.1 / 18.3).
 //  - rows of up to 4096: eight columns from 896 tiles, six and seven from 2048:
 //    14336 x 4096 N=8 17.3 / 19.1, 128256 x 4096 N=8 92 / 117, 32768 x 4096 N=6
 //    28.5 / 30.3 (13824 x 3584 N=8 and 14336 x 4096 N=6 are slower).
 //  - rows of up to 5120: seven and eight columns from 512 tiles, six too and
 //    five from 864 (13824 x 5120 N=5 21.0 / 21.7); of less than 8192: five and
-//    more from just over 8 rows per CU (3072 x 5376 N=8 12.5 / 15.0, 4096 x 6144
-//    N=6 11.9 / 13.3); of 8192: seven and eight from 512 tiles (8192 x 8192 N=8
-//    21.8 / 24.7; 28672 x 8192 N=6 51.4 against 48.9), five and more at 9 to 12
-//    rows per CU, where the column split ends (split_columns).
-static bool use_mfma_q6(int64_t M, int64_t N, int64_t K) {
+//    more from just over 8 rows per CU (3072 x 5376 N=8 12.5 / 15.0), beyond 16
+//    rows per CU where full (18944 x 6144 N=5 34.1 / 28.1, 9728 x 7680 N=6 26.7 /
+//    22.8, 9216 x 5376 N=5 18.8 / 16.1; 16384 x 6144 N=5 23.8 / 26.6); of 8192:
+//    seven and eight from 512 tiles (8192 x 8192 N=8 21.8 / 24.7; 28672 x 8192 N=6
+//    51.4 against 48.9), five and more at 9 to 12 rows per CU, where the column
+//    split ends (split_columns).
+static bool use_mfma_q6(int64_t M, int64_t N, int64_t K, int cus) {
     const int64_t tiles = (M + kMfmaRows - 1) / kMfmaRows;
+    const int fill = mfma_fill(tiles, cus);
     if (K <= 512) return N >= 3 && tiles >= 256;
-    if (K <= 3328) return (N >= (K > 3072 ? 6 : 5) && tiles >= 256) || (N == 4 && K >= 2304 && K <= 3072 && tiles >= 1024);
+    if (K < 2304) return N >= 5 && tiles >= 256 && (N > 5 || K < 2048 || fill >= 58);
+    if (K <= 3328) {
+        const bool last = K == 3328, few = tiles < 512;
+        if (N == 4) return !last && tiles >= 1024 && fill >= 80;
+        if (N < 5 || tiles < 256) return false;
+        if (N == 5) return !last && fill >= (few ? 90 : 80);
+        if (N == 6) return tiles >= 2048 || fill >= (last ? (few ? 90 : 80) : (tiles >= 1024 ? 66 : 70));
+        if (N == 7) return tiles >= 2048 || fill >= (last ? (few ? 87 : 75) : 62);
+        return !last || tiles >= 896 || fill >= 68;
+    }
     if (K <= 4096) return (N == 8 && tiles >= 896) || (N >= 6 && tiles >= 2048);
     if (K <= 5120) return (N >= 6 && tiles >= 512) || (N == 5 && tiles >= 864);
-    if (K < 8192) return N >= 5 && tiles > 128;
-    return (N >= 7 && tiles >= 512) || (K == 8192 && N >= 5 && tiles > 128 && tiles <= 192);
+    if (N < 5 || M <= 8 * cus) return false;
+    if (K < 8192) {
+        if (M <= 16 * cus) return true;
+        if (N == 5) return fill >= (K <= 6144 ? 81 : K <= 7168 ? 87 : 93);
+        if (N == 6) return fill >= (K <= 6144 ? 68 : K <= 7168 ? 75 : 81);
+        return K <= 6144 || tiles >= 512 || fill >= 68;
+    }
+    return (N >= 7 && tiles >= 512) || (K == 8192 && M <= 12 * cus);
 }
 
 // Where the pre-quantised route runs the matrix-core kernel with its A
@@ -342,13 +363,33 @@ static bool use_mfma_q6(int64_t M, int64_t N, int64_t K) {
 // caller checks) the staged matrix-core kernel is not chosen or cannot hold
 // the columns.  Measured on MI355X (us per op with a Q8_1 workspace, the
 // quantiser launch included; GA against the tile kernel or the column split):
-// 4096 x 14336 N=8 20.9 against 24.5, N=5 20.9 / 23.4, 4096 x 11008 N=5 18.3 /
-// 19.5, 8192 x 28672 N=8 55.8 / 89.9, 3072 x 14336 N=6 20.0 / 21.8, 2432 x 9472
-// N=7 15.7 / 18.4, 2934 x 22272 N=7 27.2 / 39.9; with four columns slower (4096
-// x 14336 20.8 / 20.1), and with fewer rows (1024 x 22272 N=7 25.1 / 23.9).
-static bool use_mfma_q6_ga(int64_t M, int64_t N, int64_t K) {
+// 4096 x 14336 N=8 20.9 against 24.5, 8192 x 28672 N=8 55.8 / 89.9, 3072 x 14336
+// N=6 20.0 / 21.8, 2432 x 9472 N=7 15.7 / 18.4, 2934 x 22272 N=7 27.2 / 39.9; with
+// four columns slower (4096 x 14336 20.8 / 20.1), and with fewer rows (1024 x
+// 22272 N=7 25.1 / 23.9).  Five columns of up to 16384 values, which the tile
+// kernel holds in one launch, beyond 12 rows per CU (16 to 9472 values) only where
+// full: 4096 x 11008 18.3 / 19.5, 8192 x 14336 30.9 / 33.5; not 17374 x 14848 73.1
+// / 53.1, 17584 x 9216 51.2 / 41.2, 10346 x 8448 29.2 / 25.8, 6144 x 11008 24.1 /
+// 22.9.
+static bool use_mfma_q6_ga(int64_t M, int64_t N, int64_t K, int cus) {
+    if (K <= 8192 || N < 5 || M <= 8 * cus) return false;
+    if (N > 5 || K > 16384 || M <= (K <= 9472 ? 16 : 12) * cus) return true;
     const int64_t tiles = (M + kMfmaRows - 1) / kMfmaRows;
-    return K > 8192 && N >= 5 && tiles > 128;
+    return mfma_fill(tiles, cus) >= 87 && (K <= 9472 || tiles <= 1024);
+}
+
+// Waves per workgroup of the matrix-core kernel: 8, whose staging rounds carry
+// the first loads of more items each (14336 x 4096 N=8 17.3 against 18.2 us, 3072 x
+// 5376 N=8 12.4 / 13.6, 65536 x 4096 N=8 43.7 / 44.4), or 16 for very many tiles
+// of rows of a full group (128256 x 4096 N=8 92.1 / 95.1) and, from two groups on,
+// for many tiles (65536 x 7168 N=8 90.3 / 92.4) or rounds that are not full (18944 x 7168
+// N=8 40.9 / 43.0, 35909 x 8192 N=8 74.5 / 77.7), where the columns fit beside 16 waves.
+static int q6_mfma_waves(int64_t K, int64_t M, int nc, int owaves, int cus, int max_lds) {
+    if (owaves >= 1 && owaves <= 16) return owaves > 8 ? 16 : 8;
+    const int64_t tiles = (M + kMfmaRows - 1) / kMfmaRows;
+    const bool many = K >= 3584 && K <= 4096 ? tiles > 4096
+                                             : K >= 5120 && (tiles >= 4000 || (tiles >= 1024 && mfma_fill(tiles, cus) < 65));
+    return many && q6m_lds_bytes((int)K, nc, 16) <= max_lds ? 16 : 8;
 }
 
 // The matrix-core kernel's geometry, as for Q4_K: one workgroup per CU (at
@@ -370,12 +411,7 @@ static Q6Geometry pick_geometry_q6_mfma(const DeviceInfo &di, int64_t K, int64_t
     g.rows_base = (int)(tiles / g.grid);
     g.rows_extra = (int)(tiles % g.grid);
     const int64_t nt = g.rows_base + (g.rows_extra ? 1 : 0);
-    // 8 waves, whose staging rounds carry the first loads of more items each
-    // (14336 x 4096 N=8 17.3 against 18.2 us, 3072 x 5376 N=8 12.4 / 13.6); 16
-    // for many tiles of rows of a full group (128256 x 4096 N=8 92.1 / 95.1,
-    // 64128 x 4096 53.9 / 54.4)
-    g.waves = tiles >= 4000 && K >= 3584 && K <= 4096 ? 16 : 8;
-    if (owaves >= 1 && owaves <= 16) g.waves = owaves > 8 ? 16 : 8;
+    g.waves = q6_mfma_waves(K, M, nc, owaves, cus, max_lds);
     if (ga) g.waves = 8;  // GA: its A operands in flight need more than 16 waves' registers
     const int64_t nb = K / kQK;
     g.segs = 1;
@@ -462,7 +498,7 @@ static Q6Geometry pick_geometry_q6(const DeviceInfo &di, int64_t K, int64_t M, i
     // several columns over few rows per CU: one launch of one-column channels
     // (split_columns; automatic only)
     if (fused == kFusedNone && mats == 1 && okern == 0 && g_ovr_rows.load() == 0 && g_ovr_waves.load() == 0 &&
-        g_ovr_wgs.load() == 0 && split_columns(K, M, N, cus) &&
+        g_ovr_wgs.load() == 0 && split_columns(K, M, N, cus, true) &&
         pick_geometry_q6(di, K, M, 1, N, kFusedNone, true, false).ksplit) {
         Q6Geometry g1 = pick_geometry_q6(di, K, M, 1, N, kFusedNone, f32_vec, q81);
         g1.colsplit = (int)N;
@@ -526,15 +562,17 @@ static Q6Geometry pick_geometry_q6(const DeviceInfo &di, int64_t K, int64_t M, i
     }
     // the matrix-core kernel with its A operand from the Q8_1 buffer: the
     // pre-quantised route, up to 8 columns in one launch
+    auto mfma_fits = [&](int n) {
+        return q6m_lds_bytes((int)K, n, q6_mfma_waves(K, M, n, g_ovr_waves.load(), cus, max_lds)) <= max_lds;
+    };
     if (q81 && fused == kFusedNone && mats == 1 && N <= kMfmaCols &&
-        (okern == 6 ||
-         (okern == 0 && use_mfma_q6_ga(M, N, K) &&
-          !(use_mfma_q6(M, N, K) && q6m_lds_bytes((int)K, (int)N, 16) <= max_lds))))
+        (okern == 6 || (okern == 0 && use_mfma_q6_ga(M, N, K, cus) &&
+                         !(use_mfma_q6(M, N, K, cus) && mfma_fits((int)N)))))
         return pick_geometry_q6_mfma(di, K, M, (int)N, g_ovr_wgs.load(), g_ovr_waves.load(), true);
-    if (fused == kFusedNone && mats == 1 && (okern == 4 || (okern == 0 && use_mfma_q6(M, N, K)))) {
+    if (fused == kFusedNone && mats == 1 && (okern == 4 || (okern == 0 && use_mfma_q6(M, N, K, cus)))) {
         int mc = (int)N;
-        while (mc > 1 && q6m_lds_bytes((int)K, mc, 16) > max_lds) mc = (mc + 1) / 2;
-        if (q6m_lds_bytes((int)K, mc, 16) <= max_lds && (okern == 4 || mc == N))
+        while (mc > 1 && !mfma_fits(mc)) mc = (mc + 1) / 2;
+        if (mfma_fits(mc) && (okern == 4 || mc == N))
             return pick_geometry_q6_mfma(di, K, M, mc, g_ovr_wgs.load(), g_ovr_waves.load());
     }
     int nc = (int)N;

@@ -1,9 +1,11 @@
 """The shapes on either side of the lines where the automatic choice turns to
-the matrix-core kernels: short rows, rows longer than 5120 values over few
-rows per CU, odd rows and counts that are no multiple of a tile, three to
-eight columns, both weight types.  Each against the oracle within its derived
-tolerance (every sampled output), and the F32 route against the pre-quantised
-one bit for bit, with a workspace and without."""
+the matrix-core kernels, each with the kernel that is expected there (on 256
+CUs): short rows, rounds of tiles that are full or not, rows longer than 5120
+values over few rows per CU, columns that fill the LDS, odd rows and counts that
+are no multiple of a tile, two to eight columns, both weight types.  Each
+against the oracle within its derived tolerance (every sampled output), and the
+F32 route against the pre-quantised one bit for bit, with a workspace and
+without."""
 import numpy as np
 import pytest
 
@@ -15,17 +17,33 @@ pytestmark = pytest.mark.gpu
 Q4, Q6 = 12, 14
 
 
-@pytest.mark.parametrize("wtype,M,K,N", [
-    (Q4, 4081, 256, 2), (Q4, 4080, 512, 3), (Q4, 4081, 512, 2), (Q4, 65160, 512, 7),  # one or two super-blocks
-    (Q4, 4081, 768, 5), (Q4, 4080, 1280, 8), (Q4, 4097, 3328, 6),                      # 3 to 13
-    (Q4, 16369, 2304, 4), (Q4, 16368, 2304, 4), (Q4, 32753, 3328, 3),                  # three and four columns
-    (Q4, 2049, 5376, 6), (Q4, 2048, 5376, 8), (Q4, 8177, 5888, 5),                     # long rows, staged
-    (Q4, 2049, 9472, 7), (Q4, 2048, 9472, 7), (Q4, 3001, 22272, 5),                    # A from the Q8_1 copy
-    (Q6, 4081, 512, 5), (Q6, 14333, 768, 8), (Q6, 8177, 5376, 7), (Q6, 2934, 22272, 7),
-    (Q6, 16369, 2304, 4), (Q6, 4081, 3328, 6), (Q6, 2049, 5888, 5), (Q6, 2050, 8192, 5), (Q6, 2063, 9472, 5),
-    (Q6, 4096, 512, 3),
+TILE, STAGED, SPLIT, GA = 1, 4, 5, 6  # SPLIT: K-split or one-column channels
+
+
+@pytest.mark.parametrize("wtype,M,K,N,kernel", [
+    # one or two super-blocks
+    (Q4, 4081, 256, 2, TILE), (Q4, 4593, 256, 2, STAGED), (Q4, 4080, 512, 3, TILE), (Q4, 4081, 512, 3, STAGED),
+    (Q4, 65160, 512, 7, STAGED),
+    # 3 to 13; 257 tiles of 256 CUs fill half of two rounds
+    (Q4, 4081, 768, 5, STAGED), (Q4, 4080, 1280, 8, TILE), (Q4, 4081, 3328, 6, STAGED), (Q4, 4097, 3328, 6, TILE),
+    (Q4, 6129, 2816, 5, STAGED), (Q4, 6001, 2816, 5, TILE),
+    # three and four columns
+    (Q4, 16369, 2304, 4, STAGED), (Q4, 16368, 2304, 4, TILE), (Q4, 18944, 3072, 4, TILE), (Q4, 32753, 2304, 3, STAGED), (Q4, 32753, 2816, 3, STAGED),
+    (Q4, 32753, 3072, 3, TILE),
+    # long rows: one-column channels, the tile kernel, staged
+    (Q4, 2049, 5376, 6, SPLIT), (Q4, 2048, 5376, 8, SPLIT), (Q4, 2561, 5376, 6, STAGED), (Q4, 8177, 5888, 5, STAGED),
+    (Q4, 3072, 8192, 5, SPLIT), (Q4, 2560, 6144, 5, SPLIT), (Q4, 2816, 6144, 5, TILE), (Q4, 2817, 8192, 6, SPLIT),
+    (Q4, 3585, 8192, 6, STAGED), (Q4, 4609, 8192, 6, TILE),
+    # A from the Q8_1 copy; eight columns of 14336 values beside eight waves
+    (Q4, 2049, 9472, 7, GA), (Q4, 2048, 9472, 7, SPLIT), (Q4, 3001, 22272, 5, GA), (Q4, 2560, 9472, 5, SPLIT),
+    (Q4, 2561, 9472, 5, GA), (Q4, 8177, 14336, 8, STAGED),
+    (Q6, 4081, 512, 5, STAGED), (Q6, 14333, 768, 8, STAGED), (Q6, 8177, 5376, 7, STAGED), (Q6, 2934, 22272, 7, GA),
+    (Q6, 16369, 2304, 4, STAGED), (Q6, 4081, 3328, 6, STAGED), (Q6, 2049, 5888, 5, STAGED), (Q6, 2050, 8192, 5, STAGED),
+    (Q6, 2063, 9472, 5, GA), (Q6, 4096, 512, 3, STAGED), (Q6, 4097, 9472, 5, TILE), (Q6, 6144, 5376, 5, TILE),
+    (Q6, 2048, 8192, 5, SPLIT), (Q6, 18944, 3072, 5, TILE),
 ])
-def test_choice_against_oracle_and_between_routes(Q, O, gpu, wtype, M, K, N):
+def test_choice_against_oracle_and_between_routes(Q, O, gpu, wtype, M, K, N, kernel):
+    assert Q.geometry(K, M, N, wtype)["kernel"] == kernel
     import torch
     quant = Q.quantize_rows_q4_K if wtype == Q4 else Q.quantize_rows_q6_K
     rng = np.random.default_rng(M + K + N)
@@ -41,7 +59,3 @@ def test_choice_against_oracle_and_between_routes(Q, O, gpu, wtype, M, K, N):
     assert torch.equal(Q.mul_mat_vec_q(wd, K, xd, workspace=ws, wtype=wtype), y)
     assert torch.equal(Q.op_mul_mat_vec_q(wd, K, Q.quantize_row_q8_1(xd), N, wtype=wtype), y)
 
-
-def test_staged_kernel_up_to_the_end_of_the_lds(Q, gpu):
-    """Eight columns of 14336 values fit beside eight waves (163456 of 163840 bytes)."""
-    assert Q.geometry(14336, 8192, 8)["kernel"] == 4
