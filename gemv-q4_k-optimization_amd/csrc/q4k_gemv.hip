@@ -850,6 +850,12 @@ bool split_columns(int64_t K, int64_t M, int64_t N, int cus, bool q6) {
     return rho <= lim && K <= 8 * 4096 && (K >= 4096 || ksplit_short_rows(K));
 }
 
+bool ga_in_place(int64_t K, int64_t M, int64_t N, int nc_chunk, int cus, bool q6) {
+    const bool split = M <= 12 * (int64_t)cus && K <= 8 * 4096;  // else the column split
+    const bool few = (M + kMfmaRows - 1) / kMfmaRows < 256;
+    return (few && (split || nc_chunk >= N)) || (q6 && N == 5 && K <= 16384 && nc_chunk >= N);
+}
+
 // Launch geometry for an (M, K, N) product.
 //  tile kernel: one workgroup per CU (requesting just over half the CU's LDS
 //    keeps a second one away), 8 or 16 waves, the M rows split evenly over
@@ -863,7 +869,7 @@ bool split_columns(int64_t K, int64_t M, int64_t N, int cus, bool q6) {
 //    a gate each tile pairs one row of both weights (R = 2, one or two
 //    groups in flight).
 static Geometry pick_geometry(const DeviceInfo &di, int64_t K, int64_t M, int64_t N, int fused = 0,
-                              int64_t mats = 1, bool f32_vec = true, bool q81 = false) {
+                              int64_t mats = 1, bool f32_vec = true, bool q81 = false, int mfma = kMfmaByRule) {
     Geometry g;
     const int max_lds = di.max_lds > 0 ? di.max_lds : 65536;
     const int cus = di.cus > 0 ? di.cus : 1;
@@ -874,6 +880,12 @@ static Geometry pick_geometry(const DeviceInfo &di, int64_t K, int64_t M, int64_
     const int orows = g_ovr_rows.load(), owaves = g_ovr_waves.load(), owgs = g_ovr_wgs.load();
     const int okern = g_ovr_kernel.load();
     const int rpw = bpl_rows_per_pass(K / kQK);
+    auto mfma_fits = [&](int n) { return mfma_lds_bytes((int)K, n, mfma_waves(owaves)) <= max_lds; };
+    if (mfma == kMfmaStaged) {
+        int mc = (int)N;
+        while (mc > 1 && !mfma_fits(mc)) mc = (mc + 1) / 2;
+        if (mfma_fits(mc)) return pick_geometry_mfma(di, K, M, mc, owgs, owaves);
+    }
     // several columns of rows shorter than one group: short teams (aligned
     // F32 columns, automatic only; before the column split, which these
     // shapes measured slower)
@@ -984,7 +996,6 @@ static Geometry pick_geometry(const DeviceInfo &di, int64_t K, int64_t M, int64_
     }
     // the matrix-core kernel with its A operand from the Q8_1 buffer: the
     // pre-quantised route, up to 8 columns in one launch
-    auto mfma_fits = [&](int n) { return mfma_lds_bytes((int)K, n, mfma_waves(owaves)) <= max_lds; };
     if (q81 && !fused && mats == 1 && N <= kMfmaCols &&
         (okern == 6 || (okern == 0 && use_mfma_ga(M, N, K, cus) && !(use_mfma(M, N, K, cus) && mfma_fits((int)N)))))
         return pick_geometry_mfma(di, K, M, (int)N, owgs, owaves, true);
@@ -1344,7 +1355,7 @@ static int check_weight(const void *src0, int64_t ne00, int64_t ne01, int64_t nb
 static int run_gemv(const void *src0, int64_t ne00, int64_t ne01, int64_t nb01, const float *x,
                     int64_t ldx, const uint8_t *y, int64_t stride_col_y, int64_t ncols, float *dst,
                     int64_t ld_dst, hipStream_t stream, const Epilogue *ep = nullptr,
-                    const BatchLaunch *bl = nullptr, const SumsOut *so = nullptr) {
+                    const BatchLaunch *bl = nullptr, const SumsOut *so = nullptr, int mfma = kMfmaByRule) {
     DeviceInfo *di = nullptr;
     int st = device_info(&di);
     if (st != Q4K_OK) return st;
@@ -1355,7 +1366,7 @@ static int run_gemv(const void *src0, int64_t ne00, int64_t ne01, int64_t nb01, 
     // (batched: every channel's and sample's activation 16-byte aligned too)
     const bool f32_vec = x && aligned(x, 16) && ldx % 4 == 0 &&
                          (!bl || (bl->bt.x_channel % 4 == 0 && bl->bt.x_sample % 4 == 0));
-    Geometry geo = pick_geometry(*di, ne00, ne01, ncols, fused, mats, f32_vec, !x && y);
+    Geometry geo = pick_geometry(*di, ne00, ne01, ncols, fused, mats, f32_vec, !x && y, mfma);
     if ((bl || fused || geo.colsplit) && !geo.ksplit) {  // the batched and fused tile variants: 1 or 2 slots, prologue 0 or 1
         if (fused != kFusedGate) geo.R = 1;
         if (geo.slots > 2) geo.slots = 2;
@@ -1547,6 +1558,15 @@ static int mul_mat_vec_q_q4k(const void *src0, int64_t ne00, int64_t ne01, int64
         // quantisation inside the GEMV launch (always for the K-split
         // kernels, the one route they have)
         return run_gemv(src0, ne00, ne01, nb01, src1, ldx, nullptr, 0, ne11, dst, ldd, s, nullptr, nullptr, so);
+    }
+    // no buffer for a Q8_1 copy that the product can do without (without any,
+    // where one launch holds the columns: a temporary is better than chunks)
+    if (ga_route && !ws_fits && g_ovr_kernel.load() == 0 &&
+        ga_in_place(ne00, ne01, ne11, geo.nc_chunk, di->cus, false)) {
+        const Geometry gs = pick_geometry(*di, ne00, ne01, ne11, 0, 1, true, false, kMfmaStaged);
+        if (gs.mfma && (workspace || gs.nc_chunk >= ne11))
+            return run_gemv(src0, ne00, ne01, nb01, src1, ldx, nullptr, 0, ne11, dst, ldd, s, nullptr, nullptr, so,
+                            kMfmaStaged);
     }
     // activation too large for one workgroup's LDS at this column count,
     // (with a workspace) too many values for every workgroup to quantise, or

@@ -109,6 +109,10 @@ const void *q6k_ksplit_short_kernel(int sbw, int kt, int waves, int slots, bool 
 const void *q4k_ksplit_short_nc_kernel(int nc, int sbw, int kt, int waves, int slots, bool sums, int p = 2);
 const void *q6k_ksplit_short_nc_kernel(int nc, int sbw, int kt, int waves, int slots, bool sums, int p = 2);
 
+// Which matrix-core kernels a product may take: by the rules, or the staged one
+// whatever they say (in column chunks where the columns do not fit the LDS).
+constexpr int kMfmaByRule = 0, kMfmaStaged = 1;
+
 // Q6_K weight checks and launch (q6k_gemv.hip), for the type-dispatching
 // entry points of q4k_gemv.hip.
 int check_weight_q6(const void *src0, int64_t ne00, int64_t ne01, int64_t nb01);
@@ -117,13 +121,23 @@ int check_weight_q6(const void *src0, int64_t ne00, int64_t ne01, int64_t nb01);
 int run_gemv_q6(const void *src0, int64_t ne00, int64_t ne01, int64_t nb01, const float *x, int64_t ldx,
                 const uint8_t *y, int64_t stride_col_y, int64_t ncols, float *dst, int64_t ld_dst,
                 hipStream_t stream, const Epilogue *ep = nullptr, const BatchLaunch *bl = nullptr,
-                const SumsOut *so = nullptr, int64_t geo_mats = 1);
+                const SumsOut *so = nullptr, int64_t geo_mats = 1, int mfma = kMfmaByRule);
 
 // Whether N columns of an (M, K) product run as one launch of N one-column
 // channels (q4k_gemv.hip: the measured rule), on cus CUs.
 bool split_columns(int64_t K, int64_t M, int64_t N, int cus, bool q6);
 // How full the matrix-core kernels' rounds are, in percent (q4k_gemv.hip)
 int mfma_fill(int64_t tiles, int cus);
+
+// Products that the rules give to the matrix-core kernel on a Q8_1 copy, but whose
+// F32 call needs no buffer for one: the activation fits a launch of the kernel
+// they would take otherwise (nc_chunk: the columns of its launch).  Without a
+// usable workspace they run on the staged matrix-core kernel, whose outputs are
+// the same bits, so that a call which quantises inside its launches allocates
+// nothing and takes a workspace of any size or alignment.  The others (256 row
+// tiles and more; Q6_K: but five columns of up to 16384 values) have the buffer
+// as part of their route.
+bool ga_in_place(int64_t K, int64_t M, int64_t N, int nc_chunk, int cus, bool q6);
 
 // Workgroups per weight matrix of a launch over `mats` matrices of M rows:
 // the CUs shared among the matrices, at least one, at most one per row; 16

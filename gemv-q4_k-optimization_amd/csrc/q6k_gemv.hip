@@ -478,11 +478,20 @@ static bool q6_short_nc_auto(int64_t M, int N, int nb, int cus, int &rows_per_st
 }
 
 static Q6Geometry pick_geometry_q6(const DeviceInfo &di, int64_t K, int64_t M, int64_t N, int64_t mats = 1,
-                                   int fused = kFusedNone, bool f32_vec = true, bool q81 = false) {
+                                   int fused = kFusedNone, bool f32_vec = true, bool q81 = false,
+                                   int mfma = kMfmaByRule) {
     Q6Geometry g;
     const int max_lds = di.max_lds > 0 ? di.max_lds : 65536;
     const int cus = di.cus > 0 ? di.cus : 1;
     const int okern = g_ovr_kernel.load();
+    auto mfma_fits = [&](int n) {
+        return q6m_lds_bytes((int)K, n, q6_mfma_waves(K, M, n, g_ovr_waves.load(), cus, max_lds)) <= max_lds;
+    };
+    if (mfma == kMfmaStaged) {
+        int mc = (int)N;
+        while (mc > 1 && !mfma_fits(mc)) mc = (mc + 1) / 2;
+        if (mfma_fits(mc)) return pick_geometry_q6_mfma(di, K, M, mc, g_ovr_wgs.load(), g_ovr_waves.load());
+    }
     // several columns of rows shorter than one group: short teams (aligned
     // F32 columns, the tile kernel launching all N at once; automatic only,
     // before the column split, which these shapes measured slower)
@@ -562,9 +571,6 @@ static Q6Geometry pick_geometry_q6(const DeviceInfo &di, int64_t K, int64_t M, i
     }
     // the matrix-core kernel with its A operand from the Q8_1 buffer: the
     // pre-quantised route, up to 8 columns in one launch
-    auto mfma_fits = [&](int n) {
-        return q6m_lds_bytes((int)K, n, q6_mfma_waves(K, M, n, g_ovr_waves.load(), cus, max_lds)) <= max_lds;
-    };
     if (q81 && fused == kFusedNone && mats == 1 && N <= kMfmaCols &&
         (okern == 6 || (okern == 0 && use_mfma_q6_ga(M, N, K, cus) &&
                          !(use_mfma_q6(M, N, K, cus) && mfma_fits((int)N)))))
@@ -691,7 +697,7 @@ int check_weight_q6(const void *src0, int64_t ne00, int64_t ne01, int64_t nb01) 
 int run_gemv_q6(const void *src0, int64_t ne00, int64_t ne01, int64_t nb01, const float *x, int64_t ldx,
                 const uint8_t *y, int64_t stride_col_y, int64_t ncols, float *dst, int64_t ld_dst,
                 hipStream_t stream, const Epilogue *ep, const BatchLaunch *bl, const SumsOut *so,
-                int64_t geo_mats) {
+                int64_t geo_mats, int mfma) {
     DeviceInfo *di = nullptr;
     int st = device_info(&di);
     if (st != Q4K_OK) return st;
@@ -703,7 +709,7 @@ int run_gemv_q6(const void *src0, int64_t ne00, int64_t ne01, int64_t nb01, cons
     // (batched: every channel's and sample's activation 16-byte aligned too)
     const bool f32_vec = x && aligned(x, 16) && ldx % 4 == 0 &&
                          (!bl || (bl->bt.x_channel % 4 == 0 && bl->bt.x_sample % 4 == 0));
-    const Q6Geometry geo = pick_geometry_q6(*di, ne00, ne01, ncols, mats, fused, f32_vec, !x && y);
+    const Q6Geometry geo = pick_geometry_q6(*di, ne00, ne01, ncols, mats, fused, f32_vec, !x && y, mfma);
     if (geo.colsplit) {  // the columns as one-column channels of one launch
         if (bl || fused || geo.colsplit != ncols) return Q4K_EINVAL;
         if (so) {  // parity variant: each column's launch on its own, same geometry and kernel
@@ -886,6 +892,14 @@ static int mul_mat_vec_q_q6k(const void *src0, int64_t ne00, int64_t ne01, int64
     // (the K-split kernels quantise inside the launch: their one route)
     if (geo.nc_chunk >= ne11 && !ga_route && (geo.ksplit || !(ws_fits && prefer_prequantised(ne00, ne11))))
         return run_gemv_q6(src0, ne00, ne01, nb01, src1, ldx, nullptr, 0, ne11, dst, ldd, s, nullptr, nullptr, so);
+    // no buffer for a Q8_1 copy that the product can do without, as for Q4_K
+    if (ga_route && !ws_fits && g_ovr_kernel.load() == 0 &&
+        ga_in_place(ne00, ne01, ne11, geo.nc_chunk, di->cus, true)) {
+        const Q6Geometry gs = pick_geometry_q6(*di, ne00, ne01, ne11, 1, kFusedNone, true, false, kMfmaStaged);
+        if (gs.mfma && (workspace || gs.nc_chunk >= ne11))
+            return run_gemv_q6(src0, ne00, ne01, nb01, src1, ldx, nullptr, 0, ne11, dst, ldd, s, nullptr, nullptr, so, 1,
+                               kMfmaStaged);
+    }
     // activation too large for one workgroup's LDS at this column count,
     // (with a workspace) too many values for every workgroup to quantise, or
     // the matrix-core kernel with its A operand in the Q8_1 copy:

@@ -10,11 +10,11 @@
  *
  * Memory: src0, src1 and dst are caller-owned device buffers.  Most calls
  * allocate nothing: the activation is quantised inside the GEMV launch.
- * q4k_mul_mat_vec_q and q6k_mul_mat_vec_q do allocate when the activation
- * does not fit one workgroup's LDS and no workspace is passed: a
- * stream-ordered temporary (hipMallocAsync/hipFreeAsync, the counterpart of
- * ggml's ctx.pool()) for the Q8_1 copy.  A caller with a pool (as ggml has)
- * should pass a workspace: it also speeds up several long columns.
+ * q4k_mul_mat_vec_q and q6k_mul_mat_vec_q do allocate when no workspace is
+ * passed and the product takes a Q8_1 copy (see there): a stream-ordered
+ * temporary (hipMallocAsync/hipFreeAsync, the counterpart of ggml's
+ * ctx.pool()).  A caller with a pool (as ggml has) should pass a workspace: it
+ * also speeds up several long columns.
  *
  * Threading: entry points may be called from any host thread; per-device
  * state is initialised once under a lock.  Calls that share a stream are
@@ -140,15 +140,19 @@ int q4k_quantize_row_q8_1(const float *x, void *vy, int64_t ne00, int64_t s01, i
  *   dst:  ne11 columns of ne01 floats, column stride nb1 bytes
  * ne00 must be a multiple of 256 and 1 <= ne11 <= 8 (ne01 == 0 or ne11 == 0
  * is an empty product and returns Q4K_OK).  The activation is quantised to
- * Q8_1 inside the GEMV launch when it fits one workgroup's LDS; otherwise
- * through a Q8_1 buffer: `workspace` (at least q4k_q8_1_bytes(ne00, ne11)
- * bytes, 4-B aligned) or, when NULL, a stream-ordered temporary.  With a
- * workspace of that size the buffer is also used, in a quantisation launch
- * of its own as the reference does, when ne00 * ne11 > 40960 (several long
- * columns, which every workgroup would otherwise quantise in full) and the
- * launch is not a K-split kernel (those quantise inside the launch; three or
- * four columns of 8193..16384 values run one).  Both routes give the same
- * bits. */
+ * Q8_1 inside the GEMV launch when it fits one workgroup's LDS; otherwise, and
+ * for five columns or more of rows longer than 8192 values over 4081 rows or
+ * more (q4k_gemv_geometry: out[6] is 6), through a Q8_1 buffer: `workspace`
+ * (at least q4k_q8_1_bytes(ne00, ne11) bytes, 4-B aligned, else Q4K_EINVAL) or,
+ * when NULL, a stream-ordered temporary.  With a workspace of that size the
+ * buffer is also used, in a quantisation launch of its own as the reference
+ * does, when ne00 * ne11 > 40960 (several long columns, which every workgroup
+ * would otherwise quantise in full) and the launch is not a K-split kernel
+ * (those quantise inside the launch; three or four columns of 8193..16384
+ * values run one), and for such columns over fewer rows where out[6] is 6; a
+ * workspace that is too small or not aligned is not used there, and without
+ * one the temporary is taken only where no single launch holds the columns.
+ * All routes give the same bits. */
 int q4k_mul_mat_vec_q(const void *src0, int64_t ne00, int64_t ne01, int64_t nb01,
                       const float *src1, int64_t ne11, int64_t nb11, float *dst, int64_t nb1,
                       void *workspace, size_t workspace_bytes, void *stream);
@@ -341,7 +345,8 @@ int q4k_gemv_geometry_fused(int64_t ne00, int64_t ne01, int32_t with_gate, int32
  * variant; reduced to 8 where 16 would not fit the registers), the number
  * of workgroups and the kernel (1 tile kernel, 2 block-per-lane, 3
  * coalesced block kernel where they apply, 4 matrix-core kernel for
- * products without an epilogue, 5 K-split kernel for one 16-byte aligned
+ * products without an epilogue (waves_per_wg 9..16 selects its 16-wave
+ * variant), 5 K-split kernel for one 16-byte aligned
  * F32 column of rows of up to 8 groups of 4096 values: rows_per_tile is
  * then its rows per wave step (1, 4, 8, 16; rows of other lengths than 4096
  * and 8192: 8 or 16), waves_per_wg 4, 8 or 16 (at least the rows per step;

@@ -5,7 +5,7 @@ values over few rows per CU, columns that fill the LDS, odd rows and counts that
 are no multiple of a tile, two to eight columns, both weight types.  Each
 against the oracle within its derived tolerance (every sampled output), and the
 F32 route against the pre-quantised one bit for bit, with a workspace and
-without."""
+without.  Then the calls that reach those kernels without a usable workspace."""
 import numpy as np
 import pytest
 
@@ -59,3 +59,66 @@ def test_choice_against_oracle_and_between_routes(Q, O, gpu, wtype, M, K, N, ker
     assert torch.equal(Q.mul_mat_vec_q(wd, K, xd, workspace=ws, wtype=wtype), y)
     assert torch.equal(Q.op_mul_mat_vec_q(wd, K, Q.quantize_row_q8_1(xd), N, wtype=wtype), y)
 
+
+def _weights(Q, wtype, M, K, seed):
+    quant = Q.quantize_rows_q4_K if wtype == Q4 else Q.quantize_rows_q6_K
+    wq = quant(_common.weights(min(M, 512), K, seed), nthreads=16)
+    return wq[np.random.default_rng(seed).integers(0, wq.shape[0], M)]
+
+
+def _node_types(call):
+    """The types of the graph nodes that call(stream) records (0: a kernel)."""
+    import ctypes
+    import torch
+    hip = ctypes.CDLL("libamdhip64.so")
+    stream = torch.cuda.Stream()
+    sp, graph, n = ctypes.c_void_p(stream.cuda_stream), ctypes.c_void_p(), ctypes.c_size_t(0)
+    assert hip.hipStreamBeginCapture(sp, 1) == 0  # thread-local capture mode
+    call(stream)
+    assert hip.hipStreamEndCapture(sp, ctypes.byref(graph)) == 0
+    try:
+        assert hip.hipGraphGetNodes(graph, None, ctypes.byref(n)) == 0
+        nodes = (ctypes.c_void_p * n.value)()
+        assert hip.hipGraphGetNodes(graph, nodes, ctypes.byref(n)) == 0
+        types = []
+        for nd in nodes:
+            t = ctypes.c_int(-1)
+            assert hip.hipGraphNodeGetType(ctypes.c_void_p(nd), ctypes.byref(t)) == 0
+            types.append(t.value)
+        return types
+    finally:
+        hip.hipGraphDestroy(graph)
+
+
+@pytest.mark.parametrize("wtype,M,K,N,one_launch", [
+    (Q4, 2049, 9472, 7, True), (Q4, 3001, 14336, 8, True), (Q4, 2817, 22272, 7, False), (Q4, 4080, 8448, 5, True),
+    (Q6, 2063, 9472, 5, True), (Q6, 3001, 11008, 6, True), (Q6, 2934, 22272, 7, False), (Q6, 8192, 14336, 5, True)])
+def test_no_usable_workspace(Q, O, gpu, wtype, M, K, N, one_launch):
+    """Activations that a launch can quantise by itself: a workspace that is too
+    small or not aligned is not needed, and without one the call allocates
+    nothing where one launch holds the columns.  Same bits as with one."""
+    import torch
+    assert Q.geometry(K, M, N, wtype)["kernel"] == GA
+    wd, xd = to_dev(_weights(Q, wtype, M, K, 63), gpu), to_dev(_common.activations(N, K, 64), gpu)
+    need = Q.q8_1_bytes(K, N)
+    ws = torch.empty(need, dtype=torch.uint8, device=gpu)
+    y = Q.mul_mat_vec_q(wd, K, xd, workspace=ws, wtype=wtype)
+    assert torch.equal(Q.mul_mat_vec_q(wd, K, xd, workspace=ws[: need - 4], wtype=wtype), y), "too small"
+    odd = torch.empty(need + 8, dtype=torch.uint8, device=gpu)[1:]
+    assert torch.equal(Q.mul_mat_vec_q(wd, K, xd, workspace=odd, wtype=wtype), y), "not aligned"
+    assert torch.equal(Q.mul_mat_vec_q(wd, K, xd, wtype=wtype), y), "none"
+    out = torch.empty_like(y)
+    if one_launch:
+        assert _node_types(lambda st: Q.mul_mat_vec_q(wd, K, xd, out=out, wtype=wtype, stream=st)) == [0]
+
+
+def test_workspace_that_the_route_needs(Q, gpu):
+    """256 row tiles and more of long rows: the buffer is part of the route, and one
+    that cannot hold the Q8_1 copy is refused."""
+    import torch
+    M, K, N = 4096, 14336, 6
+    assert Q.geometry(K, M, N)["kernel"] == GA
+    wd, xd = to_dev(_weights(Q, Q4, M, K, 65), gpu), to_dev(_common.activations(N, K, 66), gpu)
+    with pytest.raises(Q.Q4KError) as e:
+        Q.mul_mat_vec_q(wd, K, xd, workspace=torch.empty(Q.q8_1_bytes(K, N) - 4, dtype=torch.uint8, device=gpu))
+    assert e.value.status == Q.Q4K_EINVAL
