@@ -996,10 +996,10 @@ static Geometry pick_geometry(const DeviceInfo &di, int64_t K, int64_t M, int64_
     }
     // the matrix-core kernel with its A operand from the Q8_1 buffer: the
     // pre-quantised route, up to 8 columns in one launch
-    if (q81 && !fused && mats == 1 && N <= kMfmaCols &&
+    if (q81 && !fused && mats == 1 && N <= kMfmaCols && mfma != kMfmaNone &&
         (okern == 6 || (okern == 0 && use_mfma_ga(M, N, K, cus) && !(use_mfma(M, N, K, cus) && mfma_fits((int)N)))))
         return pick_geometry_mfma(di, K, M, (int)N, owgs, owaves, true);
-    if (!fused && mats == 1 && (okern == 4 || (okern == 0 && use_mfma(M, N, K, cus)))) {
+    if (!fused && mats == 1 && mfma != kMfmaNone && (okern == 4 || (okern == 0 && use_mfma(M, N, K, cus)))) {
         int mc = (int)N;
         while (mc > 1 && !mfma_fits(mc)) mc = (mc + 1) / 2;
         if (mfma_fits(mc) && (okern == 4 || mc == N)) return pick_geometry_mfma(di, K, M, mc, owgs, owaves);
@@ -1367,6 +1367,13 @@ static int run_gemv(const void *src0, int64_t ne00, int64_t ne01, int64_t nb01, 
     const bool f32_vec = x && aligned(x, 16) && ldx % 4 == 0 &&
                          (!bl || (bl->bt.x_channel % 4 == 0 && bl->bt.x_sample % 4 == 0));
     Geometry geo = pick_geometry(*di, ne00, ne01, ncols, fused, mats, f32_vec, !x && y, mfma);
+    // the matrix-core kernels address a workgroup's tiles with 31-bit offsets (GA:
+    // also the Q8_1 columns of a launch, as one buffer); where strides put those
+    // further apart, the kernels that address less at a time
+    const bool mfma_reach = !geo.mfma || ((int64_t)(geo.rows_base + 1) * kMfmaRows * nb01 < ((int64_t)1 << 31) &&
+                                          (!geo.mfma_ga || (int64_t)geo.nc_chunk * stride_col_y * kQ81Bytes < ((int64_t)1 << 31)));
+    if (!mfma_reach && g_ovr_kernel.load() == 0)
+        geo = pick_geometry(*di, ne00, ne01, ncols, fused, mats, f32_vec, !x && y, kMfmaNone);
     if ((bl || fused || geo.colsplit) && !geo.ksplit) {  // the batched and fused tile variants: 1 or 2 slots, prologue 0 or 1
         if (fused != kFusedGate) geo.R = 1;
         if (geo.slots > 2) geo.slots = 2;

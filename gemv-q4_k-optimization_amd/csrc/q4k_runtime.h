@@ -109,9 +109,10 @@ const void *q6k_ksplit_short_kernel(int sbw, int kt, int waves, int slots, bool 
 const void *q4k_ksplit_short_nc_kernel(int nc, int sbw, int kt, int waves, int slots, bool sums, int p = 2);
 const void *q6k_ksplit_short_nc_kernel(int nc, int sbw, int kt, int waves, int slots, bool sums, int p = 2);
 
-// Which matrix-core kernels a product may take: by the rules, or the staged one
-// whatever they say (in column chunks where the columns do not fit the LDS).
-constexpr int kMfmaByRule = 0, kMfmaStaged = 1;
+// Which matrix-core kernels a product may take: by the rules, the staged one
+// whatever they say (in column chunks where the columns do not fit the LDS), or
+// none.
+constexpr int kMfmaByRule = 0, kMfmaStaged = 1, kMfmaNone = -1;
 
 // Q6_K weight checks and launch (q6k_gemv.hip), for the type-dispatching
 // entry points of q4k_gemv.hip.

@@ -571,11 +571,12 @@ static Q6Geometry pick_geometry_q6(const DeviceInfo &di, int64_t K, int64_t M, i
     }
     // the matrix-core kernel with its A operand from the Q8_1 buffer: the
     // pre-quantised route, up to 8 columns in one launch
-    if (q81 && fused == kFusedNone && mats == 1 && N <= kMfmaCols &&
+    if (q81 && fused == kFusedNone && mats == 1 && N <= kMfmaCols && mfma != kMfmaNone &&
         (okern == 6 || (okern == 0 && use_mfma_q6_ga(M, N, K, cus) &&
                          !(use_mfma_q6(M, N, K, cus) && mfma_fits((int)N)))))
         return pick_geometry_q6_mfma(di, K, M, (int)N, g_ovr_wgs.load(), g_ovr_waves.load(), true);
-    if (fused == kFusedNone && mats == 1 && (okern == 4 || (okern == 0 && use_mfma_q6(M, N, K, cus)))) {
+    if (fused == kFusedNone && mats == 1 && mfma != kMfmaNone &&
+        (okern == 4 || (okern == 0 && use_mfma_q6(M, N, K, cus)))) {
         int mc = (int)N;
         while (mc > 1 && !mfma_fits(mc)) mc = (mc + 1) / 2;
         if (mfma_fits(mc) && (okern == 4 || mc == N))
@@ -709,7 +710,12 @@ int run_gemv_q6(const void *src0, int64_t ne00, int64_t ne01, int64_t nb01, cons
     // (batched: every channel's and sample's activation 16-byte aligned too)
     const bool f32_vec = x && aligned(x, 16) && ldx % 4 == 0 &&
                          (!bl || (bl->bt.x_channel % 4 == 0 && bl->bt.x_sample % 4 == 0));
-    const Q6Geometry geo = pick_geometry_q6(*di, ne00, ne01, ncols, mats, fused, f32_vec, !x && y, mfma);
+    Q6Geometry geo = pick_geometry_q6(*di, ne00, ne01, ncols, mats, fused, f32_vec, !x && y, mfma);
+    // (matrix-core kernels: within their offsets' reach, as for Q4_K)
+    const bool mfma_reach = !geo.mfma || ((int64_t)(geo.rows_base + 1) * kMfmaRows * nb01 < ((int64_t)1 << 31) &&
+                                          (!geo.mfma_ga || (int64_t)geo.nc_chunk * stride_col_y * kQ81Bytes < ((int64_t)1 << 31)));
+    if (!mfma_reach && g_ovr_kernel.load() == 0)
+        geo = pick_geometry_q6(*di, ne00, ne01, ncols, mats, fused, f32_vec, !x && y, kMfmaNone);
     if (geo.colsplit) {  // the columns as one-column channels of one launch
         if (bl || fused || geo.colsplit != ncols) return Q4K_EINVAL;
         if (so) {  // parity variant: each column's launch on its own, same geometry and kernel

@@ -5,7 +5,8 @@ values over few rows per CU, columns that fill the LDS, odd rows and counts that
 are no multiple of a tile, two to eight columns, both weight types.  Each
 against the oracle within its derived tolerance (every sampled output), and the
 F32 route against the pre-quantised one bit for bit, with a workspace and
-without.  Then the calls that reach those kernels without a usable workspace."""
+without.  Then the calls that reach those kernels without a usable workspace or
+with strides beyond their offsets."""
 import numpy as np
 import pytest
 
@@ -122,3 +123,27 @@ def test_workspace_that_the_route_needs(Q, gpu):
     with pytest.raises(Q.Q4KError) as e:
         Q.mul_mat_vec_q(wd, K, xd, workspace=torch.empty(Q.q8_1_bytes(K, N) - 4, dtype=torch.uint8, device=gpu))
     assert e.value.status == Q.Q4K_EINVAL
+
+
+@pytest.mark.parametrize("wtype", [Q4, Q6])
+def test_q8_1_columns_beyond_one_buffer(Q, O, gpu, wtype):
+    """Q8_1 columns so far apart that eight of them span 2^31 bytes: more than the
+    matrix-core kernel on the Q8_1 copy addresses at once, not more than the others
+    do."""
+    import torch
+    M, K, N = 3073, 8448, 8
+    assert Q.geometry(K, M, N, wtype, route="q8_1")["kernel"] == GA
+    wq = _weights(Q, wtype, M, K, 67)
+    x = _common.activations(N, K, 68)
+    wd = to_dev(wq, gpu)
+    blocks = (1 << 31) // (8 * 36) + 1
+    far = torch.empty((N, blocks, 36), dtype=torch.uint8, device=gpu)
+    q8 = Q.quantize_row_q8_1(to_dev(x, gpu)).view(N, -1, 36)[:, : K // 32]
+    far[:, : K // 32] = q8
+    dst = torch.empty((N, M), dtype=torch.float32, device=gpu)
+    name = "q4k_op_mul_mat_vec_q" if wtype == Q4 else "q6k_op_mul_mat_vec_q"
+    assert getattr(Q.lib(), name)(Q._ptr(wd), K, 0, M, Q._ptr(far), N, 32 * blocks, Q._ptr(dst), M,
+                                  Q._stream()) == Q.Q4K_OK
+    rows = np.unique(np.random.default_rng(69).choice(M, 200, replace=False))
+    ref = (O.gemv_q4K_q8_1 if wtype == Q4 else O.gemv_q6K_q8_1)(wq[rows], K, O.quantize_q8_1(x), want_sums=False)
+    _common.assert_within_tolerance(O, dst.cpu().numpy()[:, rows], ref, f"{wtype} columns far apart")
