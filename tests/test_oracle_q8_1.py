@@ -102,7 +102,7 @@ def _bounded_round_wrong(d, xs, below, above):
     quotient, the share of values that do not agree)."""
     d = np.float32(d)
     q = np.float32(xs / d)
-    q_ref = (np.sign(q) * np.floor(np.abs(q) + np.float32(0.5))).astype(np.int64) & 0xFF
+    q_ref = (np.sign(q) * np.floor(np.abs(q).astype(np.float64) + 0.5)).astype(np.int64) & 0xFF
     near = np.float32(1.0) / d
     wrong, differ = 0, 0
     for r in (near, np.nextafter(near, np.float32(0)), np.nextafter(near, np.float32(np.inf))):
