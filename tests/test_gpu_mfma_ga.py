@@ -5,10 +5,10 @@ pre-quantised route).
 
 Bar: on rows of 4096 values, where the staged matrix-core kernel also runs,
 outputs bit for bit equal to it (both sum a row's super-blocks in the same
-segments and tree, which depend on K alone); on long rows, which the staged
-kernel cannot hold in LDS, within the parity tolerance of the oracle; the
-int32 sub-block sums S_qq and the block sums S_q of q8 (formed here by a
-second MFMA against a B of ones) bit for bit against the oracle.
+segments and tree, which depend on K alone); on long rows, several of which
+the staged kernel cannot hold in LDS, within the parity tolerance of the
+oracle; the int32 sub-block sums S_qq and the block sums S_q of q8 (formed
+here by a second MFMA whose A operand is ones) bit for bit against the oracle.
 """
 import numpy as np
 import pytest

@@ -117,7 +117,7 @@ def test_q6_mfma_zero_inputs(Q, O, gpu):
 @pytest.mark.parametrize("M,K,N", [(4096, 4096, 8), (1100, 14336, 6), (2048, 768, 5)])
 def test_q6_mfma_result_independent_of_work_split(Q, O, gpu, M, K, N):
     """The summation order depends on K alone: launches over 256, 64, 16 and
-    4 workgroups, the 8-wave variant and row slices at odd offsets give the
+    4 workgroups, the 16-wave variant and row slices at odd offsets give the
     same bits."""
     import torch
     wq, x = inputs(Q, M, K, N, seed=35)
@@ -127,16 +127,17 @@ def test_q6_mfma_result_independent_of_work_split(Q, O, gpu, M, K, N):
     try:
         _force(Q)
         y = Q.mul_mat_vec_q(wd, K, xd, wtype=t6)
-        _, sums16, _ = Q.mul_mat_vec_q_sums(wd, K, xd, wtype=t6)
+        _, sums8, _ = Q.mul_mat_vec_q_sums(wd, K, xd, wtype=t6)
+        assert Q.geometry(K, M, N, t6)["waves_per_wg"] == 8
         for wgs in (64, 16, 4):
             _force(Q, workgroups=wgs)
             assert torch.equal(Q.mul_mat_vec_q(wd, K, xd, wtype=t6), y), f"{wgs} workgroups"
         for wgs in (0, 16):
-            _force(Q, waves_per_wg=8, workgroups=wgs)
-            assert Q.geometry(K, M, N, t6)["waves_per_wg"] == 8
-            assert torch.equal(Q.mul_mat_vec_q(wd, K, xd, wtype=t6), y), f"8 waves, {wgs} workgroups"
+            _force(Q, waves_per_wg=16, workgroups=wgs)
+            assert Q.geometry(K, M, N, t6)["waves_per_wg"] == 16
+            assert torch.equal(Q.mul_mat_vec_q(wd, K, xd, wtype=t6), y), f"16 waves, {wgs} workgroups"
             ys, sums, _ = Q.mul_mat_vec_q_sums(wd, K, xd, wtype=t6)
-            assert torch.equal(ys, y) and torch.equal(sums, sums16)
+            assert torch.equal(ys, y) and torch.equal(sums, sums8)
         _force(Q)
         cut = M // 3 + 5
         top = Q.op_mul_mat_vec_q(wd[:cut], K, q8d, N, row_low=0, row_high=cut, wtype=t6)
