@@ -286,8 +286,9 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q4k_ksplit_kernel(Q4K_GEMV_
 
     // the weights' requests leave before the wait for the activation: left
     // to the scheduler they sink into the quantiser (us, MI355X: 2432 x 8192
-    // 5.45 against 4.85 with this, gate 4096 x 8192 9.26 / 8.94)
-    __builtin_amdgcn_sched_barrier(0);
+    // 5.45 against 4.85 with this, gate 4096 x 8192 9.26 / 8.94; one group
+    // without a gate: no difference)
+    if constexpr (G == 2 || EPI == kEpiGlu) __builtin_amdgcn_sched_barrier(0);
 
     // 3. quantise the slice and hand each lane its sub-blocks
     LaneAct act[G];
@@ -520,7 +521,8 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q4k_ksplit_long_kernel(Q4K_
     // groups just before the step that first reads them (the first tile
     // walks the groups in order); group 0 unconditionally (a slice past the
     // row quantises zeros and writes no sums), so its load is not sunk below
-    // the weight loads
+    // the weight loads (skipped there, 1536 x 512 gains 2 % and 7324 x 512
+    // loses 4)
     uint8_t *area = lds + p.ring_off + wave * G * ks_slice_bytes(SBW);
     auto stage = [&](int i) {
         ks_stage_lds<SBW>(xv[i], lane, area + i * ks_slice_bytes(SBW), SUMS ? p.sq : nullptr,

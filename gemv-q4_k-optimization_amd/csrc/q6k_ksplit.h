@@ -167,7 +167,10 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q6k_ksplit_kernel(Q4K_GEMV_
     // 3. quantise the slice and hand each lane its groups
     Q6Act act[G];
 #pragma unroll
-    for (int i = 0; i < G; ++i) act[i] = q6_ks_stage<SBW>(xv[i], s, h, jp);
+    for (int i = 0; i < G; ++i) {
+        act[i] = q6_ks_stage<SBW>(xv[i], s, h, jp);
+        if (i + 1 < G) __builtin_amdgcn_sched_barrier(0);  // the first group does not wait for the second's values
+    }
 
     // 4. the tiles, S in flight
     int remaining = ntiles;
@@ -363,10 +366,10 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q6k_ksplit_long_kernel(Q4K_
 #pragma unroll
     for (int k = 0; k < S; ++k) load_step(st[k], w[k]);
 
-    // the weights' requests leave before the wait for the activation: left
-    // to the scheduler they sink into the quantiser (us, MI355X: 24576 x 1024
-    // 6.15 against 5.99 with this, 21248 x 1024 5.88 / 5.68)
-    __builtin_amdgcn_sched_barrier(0);
+    // short teams: the weights' requests leave before the wait for the
+    // activation (us, MI355X: 24576 x 1024 6.15 against 5.99 with this, 21248 x
+    // 1024 5.88 / 5.68)
+    if constexpr (KT > 0) __builtin_amdgcn_sched_barrier(0);
 
     // 3. quantise group 0 of the slice into the wave's LDS area, the other
     //    groups just before the step that first reads them (group 0
