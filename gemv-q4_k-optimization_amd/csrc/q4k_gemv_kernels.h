@@ -290,6 +290,9 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q4k_kernel(Q4K_GEMV_KERNEL_
     for (int k = 1; k < S; ++k) st[k] = next_step(st[k - 1], p.G);
 #pragma unroll
     for (int k = 0; k < kEarly; ++k) load_step<R, GLU>(p, ln, ws, rs_gate, st[k], w[k]);
+    // dst is loaded by now, not after the last barrier (weights from HBM: 4096 x
+    // 4096 N=4 6.27 -> 5.91 us, 9217 x 2304 N=3 7.35 -> 6.93)
+    asm volatile("" ::"s"(p.dst));
     float acc[R][NC];
 #pragma unroll
     for (int r = 0; r < R; ++r)

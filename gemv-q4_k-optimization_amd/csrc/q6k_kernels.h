@@ -330,6 +330,7 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q6k_kernel(Q4K_GEMV_KERNEL_
     for (int k = 1; k < S; ++k) st[k] = next_step(st[k - 1], p.G);
 #pragma unroll
     for (int k = 0; k < kEarly; ++k) q6_load_step<R>(p, ln, ws, st[k], w[k]);
+    asm volatile("" ::"s"(p.dst));  // dst is loaded by now, as in the Q4_K kernel
     if (p.x)
         stage_f32_finish<kLayout, kLPB, kWave * WAVES, NC < 4 ? 1 : kFinishRounds>(
             p.x, p.ldx, p.K, NC, p.vec_ok != 0, p.stage_div, xs, p.qcol, q8s, aux);
