@@ -235,13 +235,13 @@ static int tile_lds_bytes(int K, int nc, int waves) {
 }
 static int lds_bytes_linear(int K) { return K + K / 4; }
 
-// The share in percent of the matrix-core kernel's tile slots that hold a tile
-// (8 waves): a workgroup's tiles go in rounds of a power of two of them, so five
-// take the time of eight.
-int mfma_fill(int64_t tiles, int cus) {
+// The share in percent of the matrix-core kernel's tile slots that hold a tile: a
+// workgroup's tiles go in rounds of a power of two of them, up to its waves, so
+// five take the time of eight.
+int mfma_fill(int64_t tiles, int cus, int waves) {
     const int64_t nt = (tiles + cus - 1) / cus;
     int64_t groups = 1;
-    while (groups < 8 && 2 * groups <= nt) groups *= 2;
+    while (groups < waves && 2 * groups <= nt) groups *= 2;
     return (int)(100 * tiles / (cus * ((nt + groups - 1) / groups * groups)));
 }
 

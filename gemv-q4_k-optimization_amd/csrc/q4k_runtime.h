@@ -128,7 +128,7 @@ int run_gemv_q6(const void *src0, int64_t ne00, int64_t ne01, int64_t nb01, cons
 // channels (q4k_gemv.hip: the measured rule), on cus CUs.
 bool split_columns(int64_t K, int64_t M, int64_t N, int cus, bool q6);
 // How full the matrix-core kernels' rounds are, in percent (q4k_gemv.hip)
-int mfma_fill(int64_t tiles, int cus);
+int mfma_fill(int64_t tiles, int cus, int waves = 8);
 
 // Products that the rules give to the matrix-core kernel on a Q8_1 copy, but whose
 // F32 call needs no buffer for one: the activation fits a launch of the kernel

@@ -379,16 +379,19 @@ static bool use_mfma_q6_ga(int64_t M, int64_t N, int64_t K, int cus) {
 }
 
 // Waves per workgroup of the matrix-core kernel: 8, whose staging rounds carry
-// the first loads of more items each (14336 x 4096 N=8 17.3 against 18.2 us, 3072 x
-// 5376 N=8 12.4 / 13.6, 65536 x 4096 N=8 43.7 / 44.4), or 16 for very many tiles
-// of rows of a full group (128256 x 4096 N=8 92.1 / 95.1) and, from two groups on,
-// for many tiles (65536 x 7168 N=8 90.3 / 92.4) or rounds that are not full (18944 x 7168
-// N=8 40.9 / 43.0, 35909 x 8192 N=8 74.5 / 77.7), where the columns fit beside 16 waves.
+// the first loads of more items each (14336 x 4096 N=8 19.4 against 20.4 us, 3072 x
+// 5376 N=8 12.4 / 13.6, 61440 x 4096 N=8 50.5 / 51.5), or 16 where their rounds of
+// sixteen tiles are full (64128 x 4096 N=8 51.8 / 50.9, 128256 x 4096 97.0 / 94.6,
+// 62900 x 5120 63.8 / 62.0; not 73728 x 4096, 18 tiles of 32 slots, 69.6 / 78.2, nor
+// 98304 x 5120 91.1 / 105.9) and, from two groups on, where the rounds of eight are
+// little over half full (18944 x 7168 N=8 42.4 / 40.4, 35909 x 8192 82.5 / 77.8),
+// where the columns fit beside 16 waves.  Weights from HBM throughout.
 static int q6_mfma_waves(int64_t K, int64_t M, int nc, int owaves, int cus, int max_lds) {
     if (owaves >= 1 && owaves <= 16) return owaves > 8 ? 16 : 8;
     const int64_t tiles = (M + kMfmaRows - 1) / kMfmaRows;
-    const bool many = K >= 3584 && K <= 4096 ? tiles > 4096
-                                             : K >= 5120 && (tiles >= 4000 || (tiles >= 1024 && mfma_fill(tiles, cus) < 65));
+    const bool full = tiles > 15 * (int64_t)cus && mfma_fill(tiles, cus, 16) >= 94;
+    const bool many = K >= 3584 && K <= 4096 ? full
+                                             : K >= 5120 && (full || (tiles >= 1024 && mfma_fill(tiles, cus) < 65));
     return many && q6m_lds_bytes((int)K, nc, 16) <= max_lds ? 16 : 8;
 }
 
