@@ -334,6 +334,13 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q4k_ksplit_nc_long_kernel(Q
     float2 *dks = reinterpret_cast<float2 *>(lds + NC * p.qcol);
     float *part = reinterpret_cast<float *>(lds + p.ring_off);
 
+    // 1. first of all the staging loads of every wave, queued ahead of the
+    //    weight loads by the barrier below
+    constexpr int kLPB = stage_lpb(NC);
+    constexpr int kPreR = pre_rounds(NC, kWave * WAVES);
+    ActStage<kLPB, kPreR> xs;
+    stage_f32_issue<kLPB, kWave * WAVES>(p.x, p.ldx, p.K, NC, true, p.stage_div, xs);
+    __builtin_amdgcn_sched_barrier(0);
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int slice = wave % KW, team = wave / KW;
@@ -350,11 +357,6 @@ __global__ __launch_bounds__(kWave *WAVES) void gemv_q4k_ksplit_nc_long_kernel(Q
     const int kb0 = ksn_block<P, SBW>(slice, s);       // the lane's super-block within each group
     const int wkb = ksn_block<P, SBW>(slice, 0);       // the wave's first one
 
-    // 1. the staging loads of every wave, queued ahead of the weight loads
-    constexpr int kLPB = stage_lpb(NC);
-    constexpr int kPreR = pre_rounds(NC, kWave * WAVES);
-    ActStage<kLPB, kPreR> xs;
-    stage_f32_issue<kLPB, kWave * WAVES>(p.x, p.ldx, p.K, NC, true, p.stage_div, xs);
     __syncthreads();
 
     // 2. the first S steps' weights
