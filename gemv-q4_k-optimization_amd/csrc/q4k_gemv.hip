@@ -276,7 +276,10 @@ static int64_t split_rows_per_cu(int64_t N, int64_t K) {
 //    fuller): 16384 x 2304 N=4 9.33 / 10.2, 26624 x 3072 N=4 15.3 / 16.1, 24576 x
 //    2816 N=5 15.2 / 15.4, 32768 x 2304 N=3 13.0 / 14.4; not 18944 x 3072 N=4 14.6
 //    / 12.3, N=5 14.8 / 13.7, 8960 x 3328 N=5 10.6 / 9.4, 47367 x 2816 N=3 21.7 /
-//    18.6, 16526 x 3072 N=7 (half full) 15.9 / 15.2.
+//    18.6, 16526 x 3072 N=7 (half full) 15.9 / 15.2.  Of 9, where its share of the time
+//    is the smallest, less full ones too (weights from HBM): 45056 x 2304 N=4 (69 %)
+//    19.7 / 20.6, 22528 x 2304 N=5 13.2 / 14.4, 40960 x 2304 N=5 (62 %) 20.0 / 21.3; not
+//    24576 x 2304 N=4 13.0 / 12.7, 20480 x 2304 N=5 13.1 / 12.6.
 //  - rows of 16: eight columns from 896 tiles and six to eight from 4096 (14336 x
 //    4096 N=8 13.1 / 16.6, 128256 x 4096 N=8 64.6 / 87.3); with fewer rows or
 //    columns the tile kernel is within a few percent either way (4096 x 4096 N=8
@@ -298,10 +301,10 @@ static bool use_mfma(int64_t M, int64_t N, int64_t K, int cus) {
     if (K <= 512) return N >= 2 && tiles >= (N == 2 ? 288 : 256);
     if (K < 2304) return N >= 5 && tiles >= 256;
     if (K < 3584) {
-        const bool last = K == 3328;
+        const bool last = K == 3328, deep = tiles >= 10 * (int64_t)cus;  // (deep: the last round counts less)
         if (N == 3) return tiles >= 1900 && fill >= (K <= 2560 ? 87 : 93) && K <= 2816;
-        if (N == 4) return tiles >= 1024 && fill >= (last ? 93 : 80);
-        if (N == 5) return tiles >= 256 && fill >= (last ? 80 : 75);
+        if (N == 4) return tiles >= 1024 && fill >= (last ? 93 : deep && K == 2304 ? 67 : 80);
+        if (N == 5) return tiles >= 256 && fill >= (last ? 80 : K == 2304 ? (deep ? 62 : 67) : 75);
         if (N == 6) return tiles >= 256 && fill >= (last ? 75 : 65);
         if (N == 7) return tiles >= 256 && fill >= 55;
         return N == 8 && tiles >= 256;

@@ -318,7 +318,9 @@ static bool q6_ksplit_auto(int64_t K, int64_t M, int cus, int &tr, int &waves, i
 //    5.94 / 4.32).
 //  - rows of 9 to 12: the fewer columns, the fuller: 16384 x 2560 N=4 11.8 / 13.6,
 //    26624 x 2816 N=5 20.8 / 21.8, 12288 x 3072 N=6 13.4 / 14.0; not 18944 x 3072
-//    N=5 20.8 / 17.2, 6144 x 2816 N=5 9.14 / 8.67, 8768 x 3072 N=5 14.7 / 12.7.  Of
+//    N=5 20.8 / 17.2, 6144 x 2816 N=5 9.14 / 8.67, 8768 x 3072 N=5 14.7 / 12.7; from 10
+//    tiles per CU on less full ones of the shorter too (49152 x 2304 N=4 26.4 / 28.9, N=5
+//    28.4 / 32.5, 73728 x 2816 N=5 48.3 / 49.7; not N=4 45.3 / 44.2).  Of
 //    13: six and more (24576 x 3328 N=5 23.0 / 20.8; 18944 x 3328 N=6 22.1 / 18.3).
 //  - rows of up to 4096: eight columns from 896 tiles, six and seven from 2048:
 //    14336 x 4096 N=8 17.3 / 19.1, 128256 x 4096 N=8 92 / 117, 32768 x 4096 N=6
@@ -337,10 +339,10 @@ static bool use_mfma_q6(int64_t M, int64_t N, int64_t K, int cus) {
     if (K <= 512) return N >= 3 && tiles >= 256;
     if (K < 2304) return N >= 5 && tiles >= 256 && (N > 5 || K < 2048 || fill >= 58);
     if (K <= 3328) {
-        const bool last = K == 3328, few = tiles < 512;
-        if (N == 4) return !last && tiles >= 1024 && fill >= 80;
+        const bool last = K == 3328, few = tiles < 512, deep = tiles >= 10 * (int64_t)cus;
+        if (N == 4) return !last && tiles >= 1024 && fill >= (deep && K == 2304 ? 70 : 80);
         if (N < 5 || tiles < 256) return false;
-        if (N == 5) return !last && fill >= (few ? 90 : 80);
+        if (N == 5) return !last && fill >= (deep && K <= 2816 ? (K == 2304 ? 62 : 72) : few ? 90 : 80);
         if (N == 6) return tiles >= 2048 || fill >= (last ? (few ? 90 : 80) : (tiles >= 1024 ? 66 : 70));
         if (N == 7) return tiles >= 2048 || fill >= (last ? (few ? 87 : 75) : 62);
         return !last || tiles >= 896 || fill >= 68;

@@ -28,8 +28,10 @@ TILE, STAGED, SPLIT, GA = 1, 4, 5, 6  # SPLIT: K-split or one-column channels
     # 3 to 13; 257 tiles of 256 CUs fill half of two rounds
     (Q4, 4081, 768, 5, STAGED), (Q4, 4080, 1280, 8, TILE), (Q4, 4081, 3328, 6, STAGED), (Q4, 4097, 3328, 6, TILE),
     (Q4, 6129, 2816, 5, STAGED), (Q4, 6001, 2816, 5, TILE),
+    (Q4, 40960, 2304, 5, STAGED), (Q4, 20480, 2304, 5, TILE), (Q4, 45056, 2304, 4, STAGED), (Q4, 24576, 2304, 4, TILE),
     # three and four columns
-    (Q4, 16369, 2304, 4, STAGED), (Q4, 16368, 2304, 4, TILE), (Q4, 18944, 3072, 4, TILE), (Q4, 32753, 2304, 3, STAGED), (Q4, 32753, 2816, 3, STAGED),
+    (Q4, 16369, 2304, 4, STAGED), (Q4, 16368, 2304, 4, TILE), (Q4, 18944, 3072, 4, TILE), (Q4, 32753, 2304, 3, STAGED),
+    (Q4, 32753, 2816, 3, STAGED),
     (Q4, 32753, 3072, 3, TILE),
     # long rows: one-column channels, the tile kernel, staged
     (Q4, 2049, 5376, 6, SPLIT), (Q4, 2048, 5376, 8, SPLIT), (Q4, 2561, 5376, 6, STAGED), (Q4, 8177, 5888, 5, STAGED),
@@ -59,6 +61,14 @@ def test_choice_against_oracle_and_between_routes(Q, O, gpu, wtype, M, K, N, ker
     ws = torch.empty(Q.q8_1_bytes(K, N), dtype=torch.uint8, device=gpu)
     assert torch.equal(Q.mul_mat_vec_q(wd, K, xd, workspace=ws, wtype=wtype), y)
     assert torch.equal(Q.op_mul_mat_vec_q(wd, K, Q.quantize_row_q8_1(xd), N, wtype=wtype), y)
+
+
+def test_q6_waves_follow_full_rounds(Q, gpu):
+    """Q6_K takes 16 waves where their rounds of sixteen tiles are full (256 CUs)."""
+    for M, K, waves in [(64128, 4096, 16), (61440, 4096, 8), (65536, 4096, 16), (73728, 4096, 8), (98304, 5120, 8),
+                        (128256, 4096, 16), (62900, 5120, 16), (18944, 7168, 16), (14336, 4096, 8)]:
+        g = Q.geometry(K, M, 8, Q6)
+        assert (g["kernel"], g["waves_per_wg"]) == (STAGED, waves), (M, K)
 
 
 def _weights(Q, wtype, M, K, seed):
