@@ -452,11 +452,16 @@ __device__ __forceinline__ void quantize_lanes(const float (&v)[V], float &d, ui
     const float lane_max = lane_amax<true>(v);
     const float amax = block_max<LPB>(lane_max);  // (without the lanes that hold a NaN)
     d = div127(amax);
-    // (collected here, where it leaves no register across the rounding: one more
-    // than 64 took the tile kernel's second workgroup per CU, and a pre-quantised
-    // 20012 x 8448 from 22.4 to 25.2 us)
-    const bool tiny = __builtin_bit_cast(uint32_t, amax) - 1u < __builtin_bit_cast(uint32_t, 0x1p-100f) - 1u;  // but not 0
-    const uint64_t odd = __builtin_amdgcn_ballot_w64(lane_max != lane_max || tiny);
+    // 0 < amax < 2^-100, or a NaN
+    auto rare = [&] {
+        return __builtin_bit_cast(uint32_t, amax) - 1u < __builtin_bit_cast(uint32_t, 0x1p-100f) - 1u || lane_max != lane_max;
+    };
+    // four values: collected here, where it leaves no register across the
+    // rounding (one more than 64 took the tile kernel's second workgroup per CU,
+    // and a pre-quantised 20012 x 8448 from 22.4 to 25.2 us); more: with the rest,
+    // off the way to the first value (14336 x 4096 N=8 12.73 against 12.82 us)
+    uint64_t restart = 0;
+    if constexpr (V == 4) restart = __builtin_amdgcn_ballot_w64(rare());
     const float r = __builtin_amdgcn_rcpf(d);
     const float r0 = r * (1.0f - 0x1.4p-22f), r1 = r * (1.0f + 0x1.8p-22f);
     uint32_t differ[V / 4];
@@ -479,7 +484,9 @@ __device__ __forceinline__ void quantize_lanes(const float (&v)[V], float &d, ui
     uint32_t any = differ[0];
 #pragma unroll
     for (int w = 1; w < V / 4; ++w) any |= differ[w];
-    if (__builtin_expect((__builtin_amdgcn_ballot_w64(any != 0) | odd) != 0, 0)) {
+    if constexpr (V == 4) restart |= __builtin_amdgcn_ballot_w64(any != 0);
+    else restart = __builtin_amdgcn_ballot_w64(any != 0 || rare());
+    if (__builtin_expect(restart != 0, 0)) {
         const float exact_max = block_max<LPB>(lane_amax<false>(v));
         d = div127(exact_max);
         const float dd = exact_max == 0.0f ? 1.0f : d;  // (then the values are zeros and NaNs)
